@@ -1,0 +1,760 @@
+"""The work a user of libpdx has it do, as measurable cases: force evaluations and molecular
+dynamics steps of charged and uncharged systems, bead-spring melts, replica batches, and the
+learned mesh correction with its training gradient, each through the package's public entry points.
+
+``listed()`` gives the named cases, ``draw(rng)`` one more of the same ranges, ``prepare`` the
+handles and inputs a program holds before a call, ``run`` one pass, ``work`` the bytes and
+operations of a pass, ``exact`` the outputs in 64 bits from plain torch.
+"""
+import math
+import os
+import sys
+
+import numpy as np
+import torch
+
+sys.path.insert(0, os.path.join(os.getcwd(), "particledynamics.jl_amd"))
+
+import pdx  # noqa: E402
+from pdx import learned, melt, replicas, systems  # noqa: E402
+
+C_ION = 14.399645           # eV A / e^2
+A_ION = 2.82                # lattice spacing of the ionic systems (A)
+FS = 1.0 / 10.1805          # 1 fs in the A / eV / amu time unit
+KT = 300 * 8.617333e-5      # eV
+SKIN_ION = 1.0
+LJ_ION = dict(epsilon=0.01, sigma=2.8, cutoff=9.0)
+
+
+def _ions(name, sites, method="spme", spacing=1.0, order=5, rc=9.0, tol=1e-5, vacancies=0.0, jitter=0.1, lj=True,
+          energy=True, spatial=False, steps=0, mesh=0):
+    c = dict(kind="ions", nx=sites[0], ny=sites[1], nz=sites[2], method=method, spacing=spacing, order=order, rc=rc,
+             tol=tol, vacancies=vacancies, jitter=jitter, lj=lj, energy=energy, spatial=spatial, steps=steps,
+             mesh=mesh)
+    if name:
+        c["name"] = name
+    return c
+
+
+def listed():
+    return [
+        # the smallest call: one eager force and energy evaluation of the textbook LJ fluid, as a
+        # script or a minimiser makes it (launches and host work count)
+        dict(name="lj_4k_eager", kind="lj", cells=10, density=0.8442, jitter=0.05, steps=0, energy=True, graph=False),
+        # a production LJ run: 40 captured velocity-Verlet steps, a few list intervals (the row builds
+        # are part of it), forces only
+        dict(name="lj_256k_md", kind="lj", cells=40, density=0.8442, jitter=0.05, steps=40, energy=False, graph=True),
+        # a small solvated-system size with a mesh: one captured evaluation with energy and virial
+        _ions("ions_7600", (20, 20, 20), order=6, rc=10.0, mesh=40, vacancies=0.05),
+        # the ordinary ionic benchmark: 64 000 ions, LJ + smooth PME, energy and virial
+        _ions("ions_64k", (40, 40, 40)),
+        # the headline: 486 400 ions in spatial storage order, PME tuned to a 1e-4 force error
+        _ions("ions_486k", (80, 80, 80), order=6, rc=10.0, mesh=160, vacancies=0.05, spatial=True),
+        # the headline's dynamics: 40 captured velocity-Verlet steps of 1 fs at 300 K, forces only
+        _ions("ions_486k_md", (80, 80, 80), order=6, rc=10.0, mesh=160, vacancies=0.05, spatial=True, steps=40,
+              energy=False),
+        # one Coulomb force call by Ewald summation with prolates at 1e-4 (a dense mesh: many ions per node)
+        _ions("esp_64k", (40, 40, 40), method="esp", tol=1e-4, mesh=50, jitter=0.5, lj=False, energy=False),
+        # the largest force call: 512 000 ions on a sparse 300^3 smooth-PME mesh
+        _ions("spme_512k", (80, 80, 80), order=5, tol=3e-6, mesh=300, jitter=0.5, lj=False, energy=False),
+        # a bead-spring melt at production size: WCA rows and FENE bonds, energy and virial
+        dict(name="melt_1m", kind="melt", chains=10486, length=100, density=0.85, sums="fp32"),
+        # a batch of independent small boxes advanced together
+        dict(name="replicas_512", kind="replicas", boxes=512, nmin=256, nmax=8192, steps=20),
+        # the learned correction of a coarse mesh: one captured evaluation of the corrected forces
+        dict(name="learned_486k", kind="learned", sites=80, spacing=2.0, vacancies=0.05),
+        # its training: the gradient of one batch (forward and backward of the network)
+        dict(name="train_8k", kind="train", sites=30, spacing=2.0, vacancies=0.05, batch=8192),
+    ]
+
+
+def _log_int(rng, lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+def draw(rng):
+    kind = rng.choice(["lj", "ions", "ions", "ions", "ions", "melt", "replicas", "learned", "train"])
+    if kind == "lj":
+        steps = rng.choice([0, 0, rng.randint(10, 40)])
+        return dict(kind="lj", cells=_log_int(rng, 7, 40), density=round(rng.uniform(0.7, 0.9), 4),
+                    jitter=round(rng.uniform(0.02, 0.05), 4), steps=steps, energy=steps == 0 and rng.random() < 0.7,
+                    graph=steps > 0 or rng.random() < 0.5)
+    if kind == "melt":
+        length = rng.randint(20, 100)
+        return dict(kind="melt", chains=max(20, _log_int(rng, 20_000, 1_000_000) // length), length=length,
+                    density=0.85, sums=rng.choice(["fp32", "fp32", "fixed64", "fp64"]))
+    if kind == "replicas":
+        nmin = rng.randint(256, 1024)
+        return dict(kind="replicas", boxes=_log_int(rng, 8, 400), nmin=nmin, nmax=rng.randint(2 * nmin, 6000),
+                    steps=rng.randint(5, 20))
+    if kind == "learned":
+        return dict(kind="learned", sites=2 * _log_int(rng, 9, 40), spacing=round(rng.uniform(1.9, 2.4), 3),
+                    vacancies=round(rng.uniform(0.0, 0.08), 3))
+    if kind == "train":
+        return dict(kind="train", sites=2 * rng.randint(8, 15), spacing=2.0, vacancies=0.05,
+                    batch=_log_int(rng, 1000, 16384))
+    n = _log_int(rng, 9, 38)  # half the sites of a side
+    sites = [2 * max(9, min(39, n + rng.randint(-2, 2))) for _ in range(3)]
+    method = rng.choice(["spme", "spme", "spme", "p3m_ad", "p3m_ik", "esp"])
+    big = sites[0] * sites[1] * sites[2] > 250_000
+    steps = 0 if method != "spme" else rng.choice([0, 0, 0, rng.randint(10, 40)])
+    lj = method != "esp"
+    return _ions(None, sites, method=method, spacing=round(rng.uniform(1.0 if big else 0.8, 1.6), 3),
+                 order=rng.choice([4, 5, 6]) if method != "p3m_ik" else 5, rc=round(rng.uniform(8.5, 10.0), 2),
+                 tol=1e-4 if method == "esp" else rng.choice([1e-5, 3e-6]), vacancies=round(rng.uniform(0.0, 0.06), 3),
+                 jitter=round(rng.uniform(0.05, 0.1) if steps else rng.uniform(0.1, 0.4), 3), lj=lj,
+                 energy=steps == 0 and rng.random() < 0.6, spatial=rng.random() < 0.5, steps=steps)
+
+
+# ---------------------------------------------------------------- inputs
+
+
+def _rock_salt(c, seed):
+    """Rock salt of nx x ny x nz sites with neutral vacancies and Gaussian jitter: FP32 coordinates in
+    the centred box, charges, masses."""
+    n = np.array([c["nx"], c["ny"], c["nz"]])
+    L = n * A_ION
+    g = np.stack(np.meshgrid(*(np.arange(k) for k in n), indexing="ij"), -1).reshape(-1, 3)
+    q = np.where(g.sum(1) % 2 == 0, 1.0, -1.0)
+    rng = np.random.default_rng(seed)
+    k = int(round(c["vacancies"] * len(q) / 2))
+    keep = np.ones(len(q), dtype=bool)
+    if k:
+        keep[rng.choice(np.flatnonzero(q > 0), k, replace=False)] = False
+        keep[rng.choice(np.flatnonzero(q < 0), k, replace=False)] = False
+    g, q = g[keep], q[keep]
+    pos = (g + 0.25) * A_ION - L / 2 + c["jitter"] * rng.standard_normal(g.shape, dtype=np.float32)
+    pos = (pos - L * np.floor(pos / L + 0.5)).astype(np.float32)
+    L32 = L.astype(np.float32)
+    pos = np.where(pos >= L32 / 2, pos - L32, pos)
+    mass = np.where(q > 0, 22.99, 35.45)
+    v = rng.standard_normal(pos.shape) * np.sqrt(KT / mass)[:, None]
+    v -= (v * mass[:, None]).sum(0) / mass.sum()
+    return dict(pos=pos, q=q.astype(np.float32), mass=mass, vel=v.astype(np.float32), box=tuple(float(b) for b in L),
+                N=len(q))
+
+
+def _cuda(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def _columns(a):
+    return [_cuda(a[:, d]) for d in range(3)]
+
+
+def _spec(c):
+    mesh = (c["mesh"],) * 3 if c["mesh"] else None
+    kw = dict(coulomb_prefactor=C_ION, real_cutoff=c["rc"], mesh=mesh, mesh_spacing=None if mesh else c["spacing"])
+    if c["method"] == "spme":
+        return pdx.PME(real_space_tolerance=c["tol"], order=c["order"], **kw)
+    if c["method"] == "esp":
+        if mesh is None:
+            kw["mesh_spacing"] = None  # the spacing of its own rule
+        return pdx.ESP(tolerance=c["tol"], **kw)
+    return pdx.PPPM(real_space_tolerance=c["tol"], order=c["order"], differentiation=c["method"][-2:], **kw)
+
+
+def _buffers(N, energy):
+    f = [torch.zeros(N, device="cuda") for _ in range(3)]
+    if not energy:
+        return f, None, None
+    return f, torch.zeros(N, device="cuda"), torch.zeros(6, N, device="cuda")
+
+
+def _program(eng, P, q, v, energy, steps, dt, inv_mass, graph=True):
+    """What a user's program holds for repeated evaluations or steps of one system."""
+    N = P[0].numel()
+    f, E, V = _buffers(N, energy and not steps)
+    s = dict(engine=eng, P=P, q=q, f=f, E=E, V=V, energy=energy and not steps, steps=steps, graph=graph)
+    eng.evaluate(*P, q, *f, E, V, energy=s["energy"])
+    if steps:
+        s["v"] = v
+        s["start"] = [t.clone() for t in P + v + f]  # every pass advances the same initial state
+        eng.capture_step(*P, q, *v, *f, dt, inv_mass=inv_mass)
+    elif graph:
+        eng.capture(*P, q, *f, E, V, energy=energy)
+    torch.cuda.synchronize()
+    eng.status()
+    return s
+
+
+def prepare(case, seed):
+    return {"lj": _prepare_lj, "ions": _prepare_ions, "melt": _prepare_melt, "replicas": _prepare_replicas,
+            "learned": _prepare_learned, "train": _prepare_train}[case["kind"]](case, seed)
+
+
+def _lj_system(c, seed):
+    s = systems.fcc_lattice(4 * c["cells"] ** 3, c["density"], c["jitter"], seed=seed)
+    v = systems.maxwell_velocities(s["N"], 0.72, seed=seed + 1)
+    return s, v
+
+
+def _prepare_lj(c, seed):
+    s, v = _lj_system(c, seed)
+    eng = pdx.ForceEngine(s["N"], s["box"], pdx.LennardJones(1.0, 1.0, 2.5), skin=0.4)
+    P = [_cuda(s[k]) for k in "xyz"]
+    return _program(eng, P, None, _columns(v), c["energy"], c["steps"], 0.005, None, c["graph"])
+
+
+def _ion_engine(c, s, P, q, spec, correction=None, spatial=False, lj=True):
+    eng = pdx.ForceEngine(s["N"], s["box"], pdx.LennardJones(**LJ_ION) if lj else None, electrostatics=spec,
+                          charges=s["q"], skin=SKIN_ION, correction=correction, settings="auto" if spatial else None)
+    per = [_cuda(s["mass"].astype(np.float32))] + _columns(s["vel"])
+    if spatial:  # storage order made spatial once, as a production program does at set-up
+        f = [torch.zeros(s["N"], device="cuda") for _ in range(3)]
+        eng.evaluate(*P, q, *f, None, None, energy=False)
+        eng.reorder(*P, q, *per)
+    return eng, 1.0 / per[0], per[1:]
+
+
+def _prepare_ions(c, seed):
+    s = _rock_salt(c, seed)
+    P, q = _columns(s["pos"]), _cuda(s["q"])
+    eng, inv_mass, v = _ion_engine(c, s, P, q, _spec(c), spatial=c["spatial"], lj=c["lj"])
+    return _program(eng, P, q, v, c["energy"], c["steps"], FS, inv_mass)
+
+
+def _prepare_melt(c, seed):
+    s = systems.kg_chains(c["chains"], length=c["length"], density=c["density"], seed=seed)
+    X, Y, Z, bonds = melt.push_off(s, iterations=300)
+    eng = pdx.ForceEngine(s["N"], s["box"], pdx.WCA(1.0, 1.0), skin=0.4, accumulation=c["sums"], bonds=bonds,
+                          cap=2 * pdx.default_capacity(s["N"], s["box"], 2 ** (1 / 6) + 0.4))
+    st = _program(eng, [X, Y, Z], None, None, True, 0, 0.0, None)
+    st.update(box=s["box"], bonds=s["bonds"])
+    return st
+
+
+def _replica_system(c, seed):
+    """The case's batch of boxes (sizes, densities and models are the case's own), its atoms jittered
+    and given Maxwell velocities by the seed."""
+    b = systems.replica_batch(c["boxes"], seed=0, n_range=(c["nmin"], c["nmax"]))
+    rng = np.random.default_rng(seed)
+    L = np.repeat([sp["box"][0] for sp in b["specs"]], np.diff(b["offsets"]))
+    for a in "xyz":
+        r = b[a] + 0.01 * rng.standard_normal(b["N"])
+        r = (r - L * np.floor(r / L + 0.5)).astype(np.float32)
+        b[a] = np.where(r >= (L / 2).astype(np.float32), -r, r)
+        v = math.sqrt(0.72) * rng.standard_normal(b["N"])
+        v -= np.repeat(np.add.reduceat(v, b["offsets"][:-1]) / np.diff(b["offsets"]), np.diff(b["offsets"]))
+        b["v" + a] = v.astype(np.float32)
+    return b
+
+
+def _prepare_replicas(c, seed):
+    b = _replica_system(c, seed)
+    rb = pdx.ReplicaBatch(b["specs"])
+    st = replicas.device_state(b)
+    rb.forces(st, energy=False)
+    torch.cuda.synchronize()
+    return dict(batch=rb, start=st, work=replicas.clone_state(st), steps=c["steps"],
+                out=torch.zeros(c["boxes"], 4, dtype=torch.float64, device="cuda"))
+
+
+def _network(seed, feats):
+    """A network of the learned correction: its seeded weights, and the standardisation and output
+    scale (0.05 eV / A) of a residual force."""
+    mlp = learned.MLP(seed=seed % 1000)
+    mu, isd, _ = learned.fit_standardisation(feats, torch.ones(4, 3))
+    mlp.set_norm(mu, isd, 0.05)
+    return mlp
+
+
+def _coarse(c):
+    return pdx.PME(coulomb_prefactor=C_ION, real_cutoff=9.0, real_space_tolerance=1e-5, mesh_spacing=c["spacing"],
+                   order=4)
+
+
+def _learned_system(c, seed):
+    n = c["sites"]
+    return _rock_salt(dict(nx=n, ny=n, nz=n, vacancies=c["vacancies"], jitter=0.1), seed)
+
+
+def _features(c, s, rows=None):
+    P, q = _columns(s["pos"]), _cuda(s["q"])
+    sol = pdx.ElectrostaticsSolver(_coarse(c), s["box"], s["q"])
+    sol.spread(*P, q)
+    return learned.mesh_features(sol, *P, q)
+
+
+def _prepare_learned(c, seed):
+    s = _learned_system(c, seed)
+    mlp = _network(seed, _features(c, s)[:20000])
+    P, q = _columns(s["pos"]), _cuda(s["q"])
+    eng, _, _ = _ion_engine(c, s, P, q, _coarse(c), correction=mlp, spatial=True)
+    st = _program(eng, P, q, None, True, 0, 0.0, None)
+    st.update(mlp=mlp, box=s["box"])
+    return st
+
+
+def _prepare_train(c, seed):
+    s = _learned_system(c, seed)
+    feats = _features(c, s)
+    g = torch.Generator().manual_seed(seed)
+    targets = 0.05 * torch.randn(s["N"], 3, generator=g)
+    rows = torch.randint(0, s["N"], (c["batch"],), generator=g, dtype=torch.int32)
+    mlp = _network(seed, feats[:20000])
+    torch.cuda.synchronize()
+    return dict(mlp=mlp, feats=feats, targets=targets.cuda(), rows=rows.cuda())
+
+
+# ---------------------------------------------------------------- one pass
+
+
+def run(state):
+    s = state
+    if "batch" in s:
+        for k, t in s["start"].items():
+            s["work"][k].copy_(t)
+        out = s["batch"].run(s["work"], s["steps"], dt=0.005, energy=True, out=s["out"])
+        return [s["work"][k] for k in ("x", "y", "z", "vx", "vy", "vz", "fx", "fy", "fz")] + [out]
+    if "rows" in s:
+        g, loss = s["mlp"].gradient(s["feats"], s["targets"], rows=s["rows"])
+        return [g, loss]
+    eng = s["engine"]
+    if s["steps"]:
+        live = s["P"] + s["v"] + s["f"]
+        for t, t0 in zip(live, s["start"]):
+            t.copy_(t0)
+        for _ in range(s["steps"]):
+            eng.replay()
+        return live
+    if s["graph"]:
+        eng.replay()
+    else:
+        eng.evaluate(*s["P"], s["q"], *s["f"], s["E"], s["V"], energy=s["energy"])
+    out = list(s["f"])
+    if s["energy"]:
+        out += [s["E"], s["V"]]
+        if eng.solver is not None:
+            out.append(eng.Vglobal)
+    return out
+
+
+# ---------------------------------------------------------------- bytes and operations of a pass
+
+
+def _mesh_of(c, L):
+    if c.get("mesh"):
+        return (c["mesh"],) * 3
+    if c.get("method") == "esp":
+        return _spec(c).resolve_mesh(L)
+    return tuple(pdx.fft_friendly(int(math.ceil(b / c["spacing"] - 1e-9))) for b in L)
+
+
+def _mesh_flops(N, K, P, energy, fields=1):
+    nn = K[0] * K[1] * K[2]
+    fft = 2.5 * nn * math.log2(nn) * (1 + fields)
+    spread = N * (2.0 * P ** 3 + P * P)
+    gather = N * ((4.0 if fields == 1 else 6.0) * P ** 3 + 6 * P * P)
+    return fft + spread + gather + nn * (1 + (8 if energy else 0))
+
+
+def work(case):
+    """Each input read and each output written once; the operations of the pairs inside the cutoff
+    (each pair once), of the mesh's stencils and transforms, of the bonds and of the network."""
+    c = case
+    if c["kind"] == "lj":
+        N = 4 * c["cells"] ** 3
+        pairs = N * c["density"] * 4 * math.pi / 3 * 2.5 ** 3 / 2
+        if c["steps"]:  # positions, velocities and forces in and out per step
+            return dict(bytes=c["steps"] * N * 72, flops=c["steps"] * (pairs * 34 + N * 24))
+        e = c["energy"]
+        return dict(bytes=N * (12 + 12 + (28 if e else 0)), flops=pairs * (50 if e else 34))
+    if c["kind"] == "ions":
+        n = c["nx"] * c["ny"] * c["nz"]
+        N = n - 2 * int(round(c["vacancies"] * n / 2))
+        L = tuple(k * A_ION for k in (c["nx"], c["ny"], c["nz"]))
+        rho = N / (L[0] * L[1] * L[2])
+        pairs = N * rho * 4 * math.pi / 3 * c["rc"] ** 3 / 2
+        K = _mesh_of(c, L)
+        P = _spec(c).order
+        e = c["energy"] and not c["steps"]
+        mesh = _mesh_flops(N, K, P, e, 3 if c["method"] == "p3m_ik" else 1)
+        per = pairs * ((113 if e else 67) - (0 if c["lj"] else 17)) + mesh
+        if c["steps"]:
+            return dict(bytes=c["steps"] * N * 80, flops=c["steps"] * (per + N * 24))
+        return dict(bytes=N * (16 + 12 + (28 if e else 0)), flops=per)
+    if c["kind"] == "melt":
+        N = c["chains"] * c["length"]
+        return dict(bytes=N * (12 + 12 + 28 + 8), flops=N * 3.4 * 50 + N * 45)
+    if c["kind"] == "replicas":
+        atoms = c["boxes"] * (c["nmax"] - c["nmin"]) / math.log(c["nmax"] / c["nmin"])
+        per_atom = 0.8 * 2 * math.pi / 3 * (0.5 * 2.5 ** 3 + 0.5 * 2 ** 0.5) * 34 + 24
+        return dict(bytes=atoms * 72, flops=c["steps"] * atoms * per_atom)
+    if c["kind"] == "learned":
+        n = c["sites"] ** 3
+        N = n - 2 * int(round(c["vacancies"] * n / 2))
+        L = (c["sites"] * A_ION,) * 3
+        K = _mesh_of(c, L)
+        pairs = N / L[0] ** 3 * N * 4 * math.pi / 3 * 9.0 ** 3 / 2
+        mlp = N * 2.0 * (80 * 64 + 64 * 64 + 64 * 3)
+        return dict(bytes=N * 56, flops=pairs * 113 + _mesh_flops(N, K, 4, True) + mlp)
+    n = c["batch"]
+    return dict(bytes=n * (80 + 3 + 1) * 4 + 2 * 4 * learned.NPARAM, flops=6.0 * n * (80 * 64 + 64 * 64 + 64 * 3))
+
+
+# ---------------------------------------------------------------- the same in 64 bits
+
+
+def _pairs64(R, L, rc, term, want):
+    """Forces, half energies and half virials (xx, yy, zz, xy, xz, yz) of every pair closer than rc,
+    from padded cells: ``term(r2, i, j)`` gives (f, u), the force on i being f d."""
+    dev = R.device
+    N = R.shape[0]
+    Lt = torch.tensor(L, dtype=torch.float64, device=dev)
+    nc = [max(1, int(b / rc)) for b in L]
+    ncell = nc[0] * nc[1] * nc[2]
+    ijk = torch.stack([((R[:, d] / L[d] + 0.5) * nc[d]).floor().long() % nc[d] for d in range(3)], 1)
+    cell = (ijk[:, 2] * nc[1] + ijk[:, 1]) * nc[0] + ijk[:, 0]
+    order = torch.argsort(cell, stable=True)
+    count = torch.bincount(cell, minlength=ncell)
+    m = int(count.max())
+    slot = torch.arange(N, device=dev) - (count.cumsum(0) - count)[cell[order]]
+    table = torch.full((ncell, m), N, dtype=torch.long, device=dev)  # N: an empty slot
+    table[cell[order], slot] = order
+    Rp = torch.cat([R, torch.zeros(1, 3, dtype=R.dtype, device=dev)])
+    F = torch.zeros(N + 1, 3, dtype=torch.float64, device=dev)
+    E = torch.zeros(N + 1, dtype=torch.float64, device=dev)
+    V = torch.zeros(N + 1, 6, dtype=torch.float64, device=dev)
+    shifts = {(dx % nc[0], dy % nc[1], dz % nc[2]) for dx in (-1, 0, 1) for dy in (-1, 0, 1) for dz in (-1, 0, 1)}
+    step = max(1, int(2.0e7 / (m * m)))
+    for c0 in range(0, ncell, step):
+        home = torch.arange(c0, min(c0 + step, ncell), device=dev)
+        hx, hy, hz = home % nc[0], (home // nc[0]) % nc[1], home // (nc[0] * nc[1])
+        ti = table[home]
+        for sx, sy, sz in shifts:
+            other = ((hz + sz) % nc[2] * nc[1] + (hy + sy) % nc[1]) * nc[0] + (hx + sx) % nc[0]
+            tj = table[other]
+            d = Rp[ti][:, :, None, :] - Rp[tj][:, None, :, :]
+            d = d - Lt * torch.round(d / Lt)
+            r2 = (d * d).sum(-1)
+            i, j = ti[:, :, None].expand_as(r2), tj[:, None, :].expand_as(r2)
+            ok = (i < N) & (j < N) & (i != j) & (r2 < rc * rc)
+            f, u = term(torch.where(ok, r2, torch.ones_like(r2)), i.clamp_max(N - 1), j.clamp_max(N - 1))
+            f = torch.where(ok, f, torch.zeros_like(f))
+            F.index_add_(0, ti.reshape(-1), (f[..., None] * d).sum(2).reshape(-1, 3))
+            if want:
+                E.index_add_(0, ti.reshape(-1), 0.5 * torch.where(ok, u, torch.zeros_like(u)).sum(2).reshape(-1))
+                for k, (a, b) in enumerate(((0, 0), (1, 1), (2, 2), (0, 1), (0, 2), (1, 2))):
+                    V[:, k].index_add_(0, ti.reshape(-1), 0.5 * (f * d[..., a] * d[..., b]).sum(2).reshape(-1))
+    return F[:N], E[:N], V[:N]
+
+
+def _lj64(r2, eps, sigma, rc, shift):
+    s6 = (sigma * sigma / r2) ** 3
+    inside = r2 < rc * rc
+    f = 24 * eps * (2 * s6 * s6 - s6) / r2
+    u = 4 * eps * (s6 * s6 - s6) - shift
+    return torch.where(inside, f, torch.zeros_like(f)), torch.where(inside, u, torch.zeros_like(u))
+
+
+def _ewald64(R, q, L, rc, alpha, lj, want, digits=4.4):
+    """Forces, energies, half pair virials of LJ + Coulomb: real space to rc with this alpha, the whole
+    reciprocal sum (to exp(-digits^2)) as products of per-dimension phases; and its virial."""
+    dev, N = R.device, R.shape[0]
+
+    def term(r2, i, j):
+        r = r2.sqrt()
+        qq = C_ION * q[i] * q[j]
+        erfc = torch.erfc(alpha * r)
+        u = qq * erfc / r
+        f = qq * (erfc / r + 2 * alpha / math.sqrt(math.pi) * torch.exp(-alpha * alpha * r2)) / r2
+        inside = r2 < rc * rc
+        f, u = torch.where(inside, f, torch.zeros_like(f)), torch.where(inside, u, torch.zeros_like(u))
+        if lj:
+            fl, ul = _lj64(r2, LJ_ION["epsilon"], LJ_ION["sigma"], LJ_ION["cutoff"], 0.0)
+            f, u = f + fl, u + ul
+        return f, u
+
+    F, E, V = _pairs64(R, L, max(rc, LJ_ION["cutoff"] if lj else 0.0), term, want)
+    E = E - C_ION * alpha / math.sqrt(math.pi) * q * q
+    vol = L[0] * L[1] * L[2]
+    n = [int(math.ceil(2 * alpha * digits * b / (2 * math.pi))) for b in L]
+    k = [2 * math.pi / b * torch.arange(-m, m + 1, dtype=torch.float64, device=dev) for m, b in zip(n, L)]
+    k[0] = 2 * math.pi / L[0] * torch.arange(0, n[0] + 1, dtype=torch.float64, device=dev)  # half space
+    kx, ky, kz = k[0][:, None, None], k[1][None, :, None], k[2][None, None, :]
+    k2 = kx * kx + ky * ky + kz * kz
+    w = torch.full_like(k2, 2.0)
+    w[0] = 1.0
+    G = torch.where(k2 > 0, w * 4 * math.pi * C_ION / vol * torch.exp(-k2 / (4 * alpha * alpha)) / k2.clamp_min(1e-300),
+                    torch.zeros_like(k2))
+    shape = G.shape
+    S = torch.zeros(shape[0], shape[1] * shape[2], dtype=torch.complex128, device=dev)
+    step = max(64, int(4.0e7 / (shape[1] * shape[2])))
+
+    def phases(lo):
+        r = R[lo:lo + step]
+        e = [torch.exp(1j * r[:, d:d + 1] * k[d][None, :]) for d in range(3)]
+        return e[0], e[1], e[2], (e[1][:, :, None] * e[2][:, None, :]).reshape(len(r), -1)
+
+    for lo in range(0, N, step):
+        ex, _, _, eyz = phases(lo)
+        S += (ex * q[lo:lo + step, None]).T @ eyz
+    W = None
+    if want:
+        b2 = (S.real ** 2 + S.imag ** 2).reshape(shape) * G * 0.5
+        fac = 2 / k2.clamp_min(1e-300) + 1 / (2 * alpha * alpha)
+        comp = ((kx, kx), (ky, ky), (kz, kz), (kx, ky), (kx, kz), (ky, kz))
+        W = torch.stack([(b2 * ((1.0 if t < 3 else 0.0) - fac * a * b)).sum() for t, (a, b) in enumerate(comp)])
+    Q = G.reshape(S.shape) * S.conj()
+    Qx = Q * k[0][:, None]
+    for lo in range(0, N, step):
+        ex, ey, ez, eyz = phases(lo)
+        T = ((ex @ Q) * eyz).reshape(-1, shape[1], shape[2])
+        qq = q[lo:lo + step]
+        ty, tz = T.sum(2), T.sum(1)
+        E[lo:lo + step] += 0.5 * qq * ty.sum(1).real
+        F[lo:lo + step, 0] += qq * ((ex @ Qx) * eyz).sum(1).imag
+        F[lo:lo + step, 1] += qq * (ty * k[1]).sum(1).imag
+        F[lo:lo + step, 2] += qq * (tz * k[2]).sum(1).imag
+    return F, E, V, W
+
+
+def _spline64(u, P):
+    """Order-P cardinal B-spline weights and derivatives of the nodes floor(u) - P + 1 + j."""
+    t = u - u.floor()
+    M = [t, 1 - t]  # M_2(t + j)
+    for n in range(3, P + 1):
+        prev, M = M, []
+        for j in range(n):
+            left = prev[j] if j < n - 1 else torch.zeros_like(t)
+            right = prev[j - 1] if j >= 1 else torch.zeros_like(t)
+            M.append(((t + j) * left + (n - t - j) * right) / (n - 1))
+    D = [(prev[j] if j < P - 1 else 0) - (prev[j - 1] if j >= 1 else 0) for j in range(P)]
+    return (u.floor().long() - (P - 1), [M[P - 1 - j] for j in range(P)], [D[P - 1 - j] for j in range(P)])
+
+
+def _spme64(R, q, L, K, P, alpha):
+    """Smooth PME on a K mesh of order P: (charge grid, mesh forces, mesh energies, mesh virial)."""
+    dev, N = R.device, R.shape[0]
+    st = []
+    for d in range(3):
+        s = R[:, d] / L[d]
+        st.append(_spline64((s - s.floor()) * K[d], P))
+    node = [[(st[d][0] + j) % K[d] for j in range(P)] for d in range(3)]
+    grid = torch.zeros(K[2] * K[1] * K[0], dtype=torch.float64, device=dev)
+
+    def each():
+        for j3 in range(P):
+            for j2 in range(P):
+                for j1 in range(P):
+                    yield j1, j2, j3, (node[2][j3] * K[1] + node[1][j2]) * K[0] + node[0][j1]
+
+    for j1, j2, j3, at in each():
+        grid.index_add_(0, at, q * st[0][1][j1] * st[1][1][j2] * st[2][1][j3])
+    b = torch.fft.fftn(grid.reshape(K[2], K[1], K[0]))
+    m = [torch.fft.fftfreq(K[d], 1.0 / K[d], dtype=torch.float64, device=dev) for d in range(3)]
+    k = [2 * math.pi / L[d] * m[d] for d in range(3)]
+    integer = _spline64(torch.zeros(1, dtype=torch.float64), P)[1]  # M_P(P - 1 - j) at u = 0
+    dec = []
+    for d in range(3):
+        e = sum(float(integer[j]) * torch.exp(2j * math.pi * m[d] * j / K[d]) for j in range(P))
+        dec.append(1.0 / (e.real ** 2 + e.imag ** 2))
+    kx, ky, kz = k[0][None, None, :], k[1][None, :, None], k[2][:, None, None]
+    k2 = kx * kx + ky * ky + kz * kz
+    G = (4 * math.pi * C_ION / (L[0] * L[1] * L[2]) * torch.exp(-k2 / (4 * alpha * alpha)) / k2.clamp_min(1e-300)
+         * dec[0][None, None, :] * dec[1][None, :, None] * dec[2][:, None, None])
+    G[0, 0, 0] = 0.0
+    a = 0.5 * (b.real ** 2 + b.imag ** 2) * G
+    fac = 2 / k2.clamp_min(1e-300) + 1 / (2 * alpha * alpha)
+    ny = [(m[d] == -K[d] / 2) if K[d] % 2 == 0 else torch.zeros(K[d], dtype=torch.bool, device=dev) for d in range(3)]
+    ny = [ny[0][None, None, :], ny[1][None, :, None], ny[2][:, None, None]]
+    W = []
+    for t, (d, e) in enumerate(((0, 0), (1, 1), (2, 2), (0, 1), (0, 2), (1, 2))):
+        kk = (kx, ky, kz)
+        v = a * ((1.0 if t < 3 else 0.0) - fac * kk[d] * kk[e])
+        W.append((v if t < 3 else torch.where(ny[d] | ny[e], torch.zeros_like(v), v)).sum())
+    phi = (torch.fft.ifftn(b * G).real * (K[0] * K[1] * K[2])).reshape(-1)
+    E = torch.zeros(N, dtype=torch.float64, device=dev)
+    F = torch.zeros(N, 3, dtype=torch.float64, device=dev)
+    for j1, j2, j3, at in each():
+        v = phi[at]
+        w = [st[0][1][j1], st[1][1][j2], st[2][1][j3]]
+        E += 0.5 * q * v * w[0] * w[1] * w[2]
+        for d, jd in ((0, j1), (1, j2), (2, j3)):
+            o = [w[e] for e in range(3) if e != d]
+            F[:, d] -= q * v * st[d][2][jd] * o[0] * o[1] * (K[d] / L[d])
+    return grid, F, E, torch.stack(W), (st, node)
+
+
+def _weights64(mlp):
+    p = torch.from_numpy(mlp.params().astype(np.float64)).cuda()
+    out, o = [], 0
+    for shape in ((80, 64), (64,), (64, 64), (64,), (64, 3), (3,)):
+        n = int(np.prod(shape))
+        out.append(p[o:o + n].reshape(shape))
+        o += n
+    return p, out
+
+
+def _forward64(mlp, w, x):
+    mu, isd = (_cuda(a.astype(np.float64)) for a in (mlp.mu, mlp.isd))
+    h = torch.nn.functional.silu((x - mu) * isd @ w[0] + w[1])
+    return torch.nn.functional.silu(h @ w[2] + w[3]) @ w[4] + w[5]
+
+
+def _split(F):
+    return [F[:, d].contiguous() for d in range(3)]
+
+
+def exact(case, seed):
+    c = case
+    with torch.no_grad():
+        return {"lj": _exact_lj, "ions": _exact_ions, "melt": _exact_melt, "replicas": _exact_replicas,
+                "learned": _exact_learned, "train": _exact_train}[c["kind"]](c, seed)
+
+
+def _wrap64(R, Lt):
+    return R - Lt * torch.floor(R / Lt + 0.5)
+
+
+def _verlet64(R, v, inv_mass, dt, steps, force, Lt):
+    F = force(R)
+    for _ in range(steps):
+        v = v + 0.5 * dt * inv_mass * F
+        R = _wrap64(R + dt * v, Lt)
+        F = force(R)
+        v = v + 0.5 * dt * inv_mass * F
+    return _split(R) + _split(v) + _split(F)
+
+
+def _exact_lj(c, seed):
+    s, v = _lj_system(c, seed)
+    R = torch.stack([_cuda(s[k]).double() for k in "xyz"], 1)
+    Lt = torch.tensor(s["box"], dtype=torch.float64, device="cuda")
+
+    def forces(R, want=False):
+        return _pairs64(R, s["box"], 2.5, lambda r2, i, j: _lj64(r2, 1.0, 1.0, 2.5, 0.0), want)
+
+    if c["steps"]:
+        return _verlet64(R, _cuda(v).double(), 1.0, 0.005, c["steps"], lambda R: forces(R)[0], Lt)
+    F, E, V = forces(R, c["energy"])
+    return _split(F) + ([E, V.T.contiguous()] if c["energy"] else [])
+
+
+def _exact_ions(c, seed):
+    if c["steps"]:
+        return None  # an Ewald sum per step: too long
+    st = prepare(c, seed)  # the inputs in their storage order
+    spec = _spec(c)
+    R, q = torch.stack(st["P"], 1).double(), st["q"].double()
+    L = st["engine"].box
+    alpha = spec.resolved_alpha()
+    rc = c["rc"]
+    if alpha is None:  # the prolate split: the energies and forces of the whole sum do not depend on the split
+        rc = min(12.0, 0.45 * min(L))
+        alpha = 4.6 / rc
+    del st
+    F, E, V, W = _ewald64(R, q, L, rc, alpha, c["lj"], c["energy"])
+    if not c["energy"]:
+        return _split(F)
+    gaussian = spec.resolved_alpha() is not None
+    return _split(F) + [E, V.T.contiguous() if gaussian else None, W if gaussian else None]
+
+
+def _exact_melt(c, seed):
+    st = prepare(c, seed)
+    R = torch.stack(st["P"], 1).double()
+    box, bonds = st["box"], torch.from_numpy(np.asarray(st["bonds"], dtype=np.int64)).cuda()
+    del st
+    rc = 2 ** (1 / 6)
+    F, E, V = _pairs64(R, box, rc, lambda r2, i, j: _lj64(r2, 1.0, 1.0, rc, -1.0), True)
+    Lt = torch.tensor(box, dtype=torch.float64, device="cuda")
+    a, b = bonds[:, 0], bonds[:, 1]
+    d = R[a] - R[b]
+    d = d - Lt * torch.round(d / Lt)
+    r2 = (d * d).sum(1)
+    k, R02 = 30.0, 1.5 ** 2
+    f = -k / (1 - r2 / R02)
+    u = -0.5 * k * R02 * torch.log1p(-r2 / R02)
+    v = torch.stack([f * d[:, x] * d[:, y] for x, y in ((0, 0), (1, 1), (2, 2), (0, 1), (0, 2), (1, 2))], 1)
+    for i, sign in ((a, 1.0), (b, -1.0)):
+        F.index_add_(0, i, sign * f[:, None] * d)
+        E.index_add_(0, i, 0.5 * u)
+        V.index_add_(0, i, 0.5 * v)
+    return _split(F) + [E, V.T.contiguous()]
+
+
+def _exact_replicas(c, seed):
+    b = _replica_system(c, seed)
+    atoms = b["offsets"]
+    if float(((atoms[1:] - atoms[:-1]).astype(float) ** 2).sum()) * c["steps"] > 1.2e11:
+        return None
+    out = [[] for _ in range(9)]
+    summary = []
+    for k, sp in enumerate(b["specs"]):
+        lo, hi = int(atoms[k]), int(atoms[k + 1])
+        R = torch.stack([_cuda(b[a][lo:hi]).double() for a in "xyz"], 1)
+        v = torch.stack([_cuda(b["v" + a][lo:hi]).double() for a in "xyz"], 1)
+        Lt = torch.tensor(sp["box"], dtype=torch.float64, device=R.device)
+        is_lj = sp["model"] == "lj"
+        rc = 2.5 if is_lj else 2 ** (1 / 6)
+        s6 = rc ** -6.0
+        shift = 4 * (s6 * s6 - s6) if is_lj else -1.0
+        last = {}
+
+        def force(R):
+            d = R[:, None, :] - R[None, :, :]
+            d = d - Lt * torch.round(d / Lt)
+            r2 = (d * d).sum(-1)
+            r2.fill_diagonal_(1e30)
+            f, u = _lj64(r2, 1.0, 1.0, rc, shift)
+            last.update(u=0.5 * u.sum(), w=0.5 * (f * r2).sum())
+            return (f[..., None] * d).sum(1)
+
+        res = _verlet64(R, v, 1.0, 0.005, c["steps"], force, Lt)
+        for o, r in zip(out, res):
+            o.append(r)
+        kin = 0.5 * sum((a * a).sum() for a in res[3:6])
+        summary.append(torch.stack([last["u"], kin, last["w"], last["u"].new_tensor(float(hi - lo))]))
+    return [torch.cat(o) for o in out] + [torch.stack(summary)]
+
+
+def _exact_learned(c, seed):
+    st = prepare(c, seed)
+    spec = _coarse(c)
+    R, q = torch.stack(st["P"], 1).double(), st["q"].double()
+    eng, mlp, L = st["engine"], st["mlp"], st["box"]
+    K, alpha = eng.solver.mesh, spec.resolved_alpha()
+
+    def term(r2, i, j):
+        r = r2.sqrt()
+        qq = C_ION * q[i] * q[j]
+        erfc = torch.erfc(alpha * r)
+        f = qq * (erfc / r + 2 * alpha / math.sqrt(math.pi) * torch.exp(-alpha * alpha * r2)) / r2
+        fl, ul = _lj64(r2, LJ_ION["epsilon"], LJ_ION["sigma"], LJ_ION["cutoff"], 0.0)
+        return f + fl, qq * erfc / r + ul
+
+    F, E, V = _pairs64(R, L, 9.0, term, True)
+    E = E - C_ION * alpha / math.sqrt(math.pi) * q * q
+    grid, Fm, Em, W, (sp, node) = _spme64(R, q, L, K, 4, alpha)
+    x = torch.zeros(len(q), 80, dtype=torch.float64, device="cuda")
+    for j3 in range(4):
+        for j2 in range(4):
+            for j1 in range(4):
+                x[:, 16 * j3 + 4 * j2 + j1] = q * grid[(node[2][j3] * K[1] + node[1][j2]) * K[0] + node[0][j1]]
+    for d in range(3):
+        s = R[:, d] / L[d]
+        u = (s - s.floor()) * K[d]
+        x[:, 64 + d] = q * (u - u.floor())
+    x[:, 67], x[:, 68] = q, q * q
+    _, w = _weights64(mlp)
+    F = F + Fm + mlp.out_scale * _forward64(mlp, w, x)
+    return _split(F) + [E + Em, V.T.contiguous(), W]
+
+
+def _exact_train(c, seed):
+    st = prepare(c, seed)
+    rows = st["rows"].long()
+    x, t = st["feats"][rows].double(), st["targets"][rows].double()
+    p, _ = _weights64(st["mlp"])
+    with torch.enable_grad():
+        p = p.requires_grad_(True)
+        w, o = [], 0
+        for shape in ((80, 64), (64,), (64, 64), (64,), (64, 3), (3,)):
+            n = int(np.prod(shape))
+            w.append(p[o:o + n].reshape(shape))
+            o += n
+        loss = ((_forward64(st["mlp"], w, x) - t / st["mlp"].out_scale) ** 2).mean()
+        g, = torch.autograd.grad(loss, p)
+    return [g, loss.detach().reshape(1)]
