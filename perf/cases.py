@@ -169,8 +169,10 @@ def _program(eng, P, q, v, energy, steps, dt, inv_mass, graph=True):
     eng.evaluate(*P, q, *f, E, V, energy=s["energy"])
     if steps:
         s["v"] = v
-        s["start"] = [t.clone() for t in P + v + f]  # every pass advances the same initial state
+        v0 = [t.clone() for t in P + v + f]
         eng.capture_step(*P, q, *v, *f, dt, inv_mass=inv_mass)
+        for t, t0 in zip(P + v + f, v0):  # the capture's warm-up step is undone: step 1 is the first replay
+            t.copy_(t0)
     elif graph:
         eng.capture(*P, q, *f, E, V, energy=energy)
     torch.cuda.synchronize()
@@ -312,12 +314,9 @@ def run(state):
         return [g, loss]
     eng = s["engine"]
     if s["steps"]:
-        live = s["P"] + s["v"] + s["f"]
-        for t, t0 in zip(live, s["start"]):
-            t.copy_(t0)
-        for _ in range(s["steps"]):
+        for _ in range(s["steps"]):  # the next pass goes on from here, as a run does
             eng.replay()
-        return live
+        return s["P"] + s["v"] + s["f"]
     if s["graph"]:
         eng.replay()
     else:
