@@ -24,6 +24,7 @@ FS = 1.0 / 10.1805          # 1 fs in the A / eV / amu time unit
 KT = 300 * 8.617333e-5      # eV
 SKIN_ION = 1.0
 LJ_ION = dict(epsilon=0.01, sigma=2.8, cutoff=9.0)
+LJ_ION_MD = dict(epsilon=0.01, sigma=3.17, cutoff=9.0)  # the lattice spacing is its equilibrium: it stays a solid
 
 
 def _ions(name, sites, method="spme", spacing=1.0, order=5, rc=9.0, tol=1e-5, vacancies=0.0, jitter=0.1, lj=True,
@@ -165,7 +166,7 @@ def _program(eng, P, q, v, energy, steps, dt, inv_mass, graph=True):
     """What a user's program holds for repeated evaluations or steps of one system."""
     N = P[0].numel()
     f, E, V = _buffers(N, energy and not steps)
-    s = dict(engine=eng, P=P, q=q, f=f, E=E, V=V, energy=energy and not steps, steps=steps, graph=graph)
+    s = dict(engine=eng, P=P, q=q, f=f, E=E, V=V, energy=energy and not steps, steps=steps, graph=graph, im=inv_mass)
     eng.evaluate(*P, q, *f, E, V, energy=s["energy"])
     if steps:
         s["v"] = v
@@ -198,8 +199,9 @@ def _prepare_lj(c, seed):
     return _program(eng, P, None, _columns(v), c["energy"], c["steps"], 0.005, None, c["graph"])
 
 
-def _ion_engine(c, s, P, q, spec, correction=None, spatial=False, lj=True):
-    eng = pdx.ForceEngine(s["N"], s["box"], pdx.LennardJones(**LJ_ION) if lj else None, electrostatics=spec,
+def _ion_engine(c, s, P, q, spec, correction=None, spatial=False, lj=True, steps=0):
+    model = pdx.LennardJones(**(LJ_ION_MD if steps else LJ_ION)) if lj else None
+    eng = pdx.ForceEngine(s["N"], s["box"], model, electrostatics=spec,
                           charges=s["q"], skin=SKIN_ION, correction=correction, settings="auto" if spatial else None)
     per = [_cuda(s["mass"].astype(np.float32))] + _columns(s["vel"])
     if spatial:  # storage order made spatial once, as a production program does at set-up
@@ -212,7 +214,8 @@ def _ion_engine(c, s, P, q, spec, correction=None, spatial=False, lj=True):
 def _prepare_ions(c, seed):
     s = _rock_salt(c, seed)
     P, q = _columns(s["pos"]), _cuda(s["q"])
-    eng, inv_mass, v = _ion_engine(c, s, P, q, _spec(c), spatial=c["spatial"], lj=c["lj"])
+    eng, inv_mass, v = _ion_engine(c, s, P, q, _spec(c), spatial=c["spatial"], lj=c["lj"],
+                                   steps=c["steps"])
     return _program(eng, P, q, v, c["energy"], c["steps"], FS, inv_mass)
 
 
