@@ -143,6 +143,11 @@ __device__ __forceinline__ int wave_max(int v) {
   for (int off = 32; off >= 1; off >>= 1) v = max(v, __shfl_xor(v, off, WAVE));
   return v;
 }
+__device__ __forceinline__ int wave_min(int v) {
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) v = min(v, __shfl_xor(v, off, WAVE));
+  return v;
+}
 __device__ __forceinline__ float wave_max(float v) {
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, WAVE));
@@ -164,6 +169,29 @@ __device__ void block_partials(const double (&v)[NV], double *partial) {
 #pragma unroll
   for (int c = 0; c < NV; ++c) {
     double s = wave_sum(v[c]);
+    if (lane == 0) sh[c][wave] = s;
+  }
+  __syncthreads();
+  if (threadIdx.x < NV) {
+    double s = 0.0;
+    for (int w = 0; w < nwave; ++w) s += sh[threadIdx.x][w];
+    partial[(size_t)blockIdx.x * NV + threadIdx.x] = s;
+  }
+}
+
+// block_partials for values that only every STEP-th lane holds (the other lanes pass zeros): the
+// wave sums skip the log2(STEP) exchanges that would only add zeros.
+template <int NV, int STEP>
+__device__ void block_partials_every(const double (&v)[NV], double *partial) {
+  __shared__ double sh[NV][16];
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wave = threadIdx.x / WAVE;
+  const int nwave = blockDim.x / WAVE;
+#pragma unroll
+  for (int c = 0; c < NV; ++c) {
+    double s = v[c];
+#pragma unroll
+    for (int off = 32; off >= STEP; off >>= 1) s += __shfl_xor(s, off, WAVE);
     if (lane == 0) sh[c][wave] = s;
   }
   __syncthreads();

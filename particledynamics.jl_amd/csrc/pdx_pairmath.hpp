@@ -103,4 +103,47 @@ __device__ __forceinline__ void pair_terms(const A &a, const float (&pe)[NP], co
   pair_terms_c<MODEL, COUL, ENERGY, NP>(a, c, pe, pf, qi, qj, r2, f, u);
 }
 
+// pair_terms with the masks on the factors (1/r, (sigma/r)^6, the charge product) instead of the
+// finished terms, so that force and energy share them, and the Coulomb terms joined by fused steps:
+// about seven instructions fewer per visit with energies, equal to pair_terms up to FP32 rounding.
+// pe[0] carries the cutoff energy shift (-ceshift). A: the fields of pair_terms.
+template <int MODEL, bool COUL, bool ENERGY, int NP, typename A>
+__device__ __forceinline__ void pair_terms_joint(const A &a, const float (&pe)[NP], const float (&pf)[NP], float cqi,
+                                                 float qj, float r2, float &f, float &u) {
+  f = 0.f;
+  u = 0.f;
+  const bool pos = r2 > 0.f;
+  const bool in = pos & (r2 < a.rc2);
+  float rinv = 0.f, i2;
+  if (COUL) {
+    rinv = pos ? __builtin_amdgcn_rsqf(r2) : 0.f;
+    i2 = rinv * rinv;
+  } else {
+    i2 = in ? __builtin_amdgcn_rcpf(r2) : 0.f;
+  }
+  if (lj_form(MODEL)) {
+    const float s2 = a.sig2 * i2;
+    float s6 = s2 * s2 * s2;
+    if (COUL) s6 = in ? s6 : 0.f;
+    const float t = fmaf(s6, s6, -s6);
+    f = (24.0f * a.eps) * fmaf(s6, s6, t) * i2;
+    if (ENERGY) {
+      const float ul = fmaf(4.0f * a.eps, t, wca_energy(MODEL) ? a.eps : -a.eshift);
+      u = in ? ul : 0.f;
+    }
+  } else if (MODEL == PDX_PAIR_SOFT) {
+    const float r = sqrtf(r2);
+    const float sg = sqrtf(a.sig2);
+    const float xx = 1.0f - r / sg;
+    f = in ? (a.eps / sg) * xx / r : 0.f;
+    if (ENERGY) u = in ? 0.5f * a.eps * xx * xx : 0.f;
+  }
+  if (COUL) {
+    const float x = fmaf(r2, a.csx, -1.0f);
+    const float cq = (pos & (r2 < a.crc2)) ? cqi * qj : 0.f;
+    f = fmaf(cq, fmaf(rinv, i2, -horner<NP>(pf, x)), f);
+    if (ENERGY) u = fmaf(cq, rinv + horner<NP>(pe, x), u);
+  }
+}
+
 }  // namespace pdx
