@@ -2,8 +2,6 @@
 // in one persistent launch: one workgroup owns one replica for every step, so replicas never
 // synchronise with each other and a step costs no kernel launch. Per step, inside the
 // workgroup:
-//   A  kick-drift v += c f, x += dt v, wrap to [-L/2, L/2) (_nve_kick_drift3_kernel!,
-//      src/simulation/NVEFusion.jl:3-24), cell of each atom, LDS histogram;
 //   B  exclusive scan of the cell counts (LDS);
 //   C  scatter (x, y, z, id) into cell order in LDS;
 //   D  each cell's slice put in atom-id order (stable order: the traversal, and with it the
@@ -11,9 +9,17 @@
 //   E  forces from the LDS-resident sorted coordinates over the (2S+1)^3 stencil of cells of
 //      side >= rc/S (or over all atoms for boxes with fewer than 2S+1 cells a side, as the
 //      reference's all-pairs rows, DenseNeighborCUDA.jl:128-151), then the closing kick
-//      v += c f (_nve_kick3_kernel!, src/SimulationCore.jl:581-591).
-// Atom state (x, v, f) stays in HBM / L2 between phases; the sorted coordinates and the
-// cell table live in LDS (up to 8192 atoms: 128 KiB of float4, within gfx950's 160 KiB).
+//      v += c f (_nve_kick3_kernel!, src/SimulationCore.jl:581-591), the next step's kick-drift
+//      v += c f, x += dt v, wrap to [-L/2, L/2) (_nve_kick_drift3_kernel!,
+//      src/simulation/NVEFusion.jl:3-24) and the drifted atom's cell count.
+// Atom state (x, v) stays in HBM / L2 between phases; the sorted coordinates, the cell table and
+// the next counts live in LDS (up to 8192 atoms: 128 KiB of float4, within gfx950's 160 KiB).
+// The launch lasts as long as its largest replica, one workgroup alone on its CU (its coordinates
+// fill the LDS) and bound by VALU issue in E, so E visits few candidates and spends little on each:
+// a stencil is walked as (2S+1)^2 rows of cells, contiguous in LDS; a row further than rc is left
+// out and the others are cut to the cells a sphere of rc reaches; a row's image shift is subtracted
+// from the atom once instead of testing every pair. 512 boxes of 256..8192 atoms, 20 steps: 31.0 ms
+// with 27-cell stencils, a separate kick-drift pass and 512 threads, 8.6 ms now (0.43 ms a step).
 #include "pdx_internal.hpp"
 
 #include <algorithm>
@@ -26,7 +32,7 @@ using namespace pdx;
 namespace {
 
 constexpr int NMAX = 8192;   // atoms per replica (LDS-resident sorted coordinates)
-constexpr int NCMAX = 8192;  // cells per replica
+constexpr int NCMAX = 6000;  // cells per replica (their 16-bit starts and counts, 24 KiB, fit beside NMAX atoms)
 constexpr int RED_BYTES = 1024;
 
 struct Rep {
@@ -34,7 +40,8 @@ struct Rep {
   int model;     // PDX_PAIR_LJ / PDX_PAIR_WCA
   int S;         // stencil half-width in cells; 0: all pairs
   int nc[3];     // cells per dimension
-  float L[3], halfL[3], cinv[3];  // box, half box, cells per unit length
+  float L[3], halfL[3], cinv[3], cw[3];  // box, half box, cells per unit length, cell width
+  float slack;                           // bound of the rounding of a cell edge
   float eps, sig2, rc2, eshift;
 };
 
@@ -73,18 +80,99 @@ __device__ __forceinline__ double block_sum(double v, double *red) {
   return s;
 }
 
+// Lanes per atom of the force phase: small replicas would leave most of the workgroup idle. A
+// function of n alone, as the lanes' partial sums are part of the replica's arithmetic.
+__host__ __device__ inline int atom_lanes(int n) { return n <= 512 ? 4 : (n <= 1024 ? 2 : 1); }
+
+// Forces on the atom at p (slot s): its share (rows sub, sub + G, ...) of the stencil's rows of cells,
+// in row order, every row in x order. ENERGY also sums the pair energies and r.F.
+template <bool ENERGY>
+__device__ __forceinline__ void atom_forces(const Rep &R, const float4 *spos, const unsigned short *cst, int n,
+                                            const float4 &p, int s, int sub, int G, float &ax, float &ay, float &az,
+                                            float &e, float &w) {
+  auto pair = [&](float dx, float dy, float dz) {
+    const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+    float f, u;
+    lj_terms(R, r2, f, u);
+    ax = fmaf(f, dx, ax); ay = fmaf(f, dy, ay); az = fmaf(f, dz, az);
+    if (ENERGY) {
+      e += u;
+      w = fmaf(f, r2, w);
+    }
+  };
+  if (R.S == 0) {
+    for (int j = sub; j < n; j += G) {
+      const float4 q = spos[j];
+      pair(mic_fast(p.x - q.x, R.halfL[0], R.L[0]), mic_fast(p.y - q.y, R.halfL[1], R.L[1]),
+           mic_fast(p.z - q.z, R.halfL[2], R.L[2]));
+    }
+    return;
+  }
+  const int S = R.S;
+  const int nx = R.nc[0], ny = R.nc[1], nz = R.nc[2];
+  const int cx = cell_coord(p.x, R.halfL[0], R.cinv[0], nx);
+  const int cy = cell_coord(p.y, R.halfL[1], R.cinv[1], ny);
+  const int cz = cell_coord(p.z, R.halfL[2], R.cinv[2], nz);
+  const float ux = p.x + R.halfL[0];
+  int r = 0;
+  for (int oz = -S; oz <= S; ++oz) {
+    // a row's distance from the atom in z and y, less a slack that covers the rounding of the edges
+    const float gz = (float)(cz + oz) * R.cw[2] - R.halfL[2];
+    float dz = oz > 0 ? gz - p.z : (oz < 0 ? p.z - (gz + R.cw[2]) : 0.f);
+    dz = fmaxf(dz - R.slack, 0.f);
+    const float remz = fmaf(-dz, dz, R.rc2);
+    int z2 = cz + oz;
+    float pz = p.z;
+    if (z2 < 0) { z2 += nz; pz += R.L[2]; } else if (z2 >= nz) { z2 -= nz; pz -= R.L[2]; }
+    for (int oy = -S; oy <= S; ++oy, ++r) {
+      if (G > 1 && (r & (G - 1)) != sub) continue;
+      const float gy = (float)(cy + oy) * R.cw[1] - R.halfL[1];
+      float dy = oy > 0 ? gy - p.y : (oy < 0 ? p.y - (gy + R.cw[1]) : 0.f);
+      dy = fmaxf(dy - R.slack, 0.f);
+      const float rem = fmaf(-dy, dy, remz);
+      if (!(rem > 0.f)) continue;
+      const float xr = __builtin_amdgcn_sqrtf(rem) + R.slack;  // (its ulp is within the slack)
+      const int x0 = max((int)floorf((ux - xr) * R.cinv[0]), cx - S);
+      const int x1 = min((int)floorf((ux + xr) * R.cinv[0]), cx + S);
+      int y2 = cy + oy;
+      float py = p.y;
+      if (y2 < 0) { y2 += ny; py += R.L[1]; } else if (y2 >= ny) { y2 -= ny; py -= R.L[1]; }
+      // cells x0..x1 of the row as at most two runs of slots, one per image; one loop over both, as
+      // most waves hold atoms at both ends of a row. An odd last step pairs the atom with itself.
+      const unsigned short *cs = cst + (z2 * ny + y2) * nx;
+      const bool left = x0 < 0, right = x1 >= nx;
+      const float p0 = left ? p.x + R.L[0] : p.x, p1 = left ? p.x : p.x - R.L[0];
+      const int b0 = cs[left ? x0 + nx : x0], l0 = (int)cs[left || right ? nx : x1 + 1] - b0;
+      int b1 = 0, tot = l0;
+      if (left | right) {
+        b1 = cs[0];
+        tot += (int)cs[(left ? x1 : x1 - nx) + 1] - b1;
+        b1 -= l0;
+      }
+      for (int k = 0; k < tot; k += 2) {
+        const bool i0 = k < l0, i1 = k + 1 < l0;
+        const float4 q0 = spos[k + (i0 ? b0 : b1)];
+        const float4 q1 = spos[k + 1 < tot ? k + 1 + (i1 ? b0 : b1) : s];
+        pair((i0 ? p0 : p1) - q0.x, py - q0.y, pz - q0.z);
+        pair((i1 ? p0 : p1) - q1.x, py - q1.y, pz - q1.z);
+      }
+    }
+  }
+}
+
 template <int BS>
 __global__ __launch_bounds__(BS) void k_replicas(const Rep *__restrict__ reps, const int32_t *__restrict__ order,
                                                  float *x, float *y, float *z, float *vx, float *vy, float *vz,
                                                  float *fx, float *fy, float *fz, int32_t *key, float c, float dt,
                                                  float mass, int nsteps, int first_force, int energy, int reg0,
-                                                 int reg1, double *out) {
+                                                 int reg1, int reg2, double *out) {
   extern __shared__ float4 smem[];
   float4 *spos = smem;
-  int *cnt = reinterpret_cast<int *>(smem);  // aliases spos while binning
-  unsigned short *cst = reinterpret_cast<unsigned short *>(reinterpret_cast<char *>(smem) + reg0);
-  int *wsum = reinterpret_cast<int *>(reinterpret_cast<char *>(smem) + reg0 + reg1);
-  double *red = reinterpret_cast<double *>(reinterpret_cast<char *>(smem) + reg0 + reg1 + 128);
+  char *base0 = reinterpret_cast<char *>(smem) + reg0;
+  unsigned short *cst = reinterpret_cast<unsigned short *>(base0);     // cell starts
+  unsigned *cnt = reinterpret_cast<unsigned *>(base0 + reg1);          // next counts, two 16-bit cells a word
+  int *wsum = reinterpret_cast<int *>(base0 + reg1 + reg2);
+  double *red = reinterpret_cast<double *>(base0 + reg1 + reg2 + 128);
 
   const int rid = order[blockIdx.x];
   const Rep R = reps[rid];
@@ -93,41 +181,46 @@ __global__ __launch_bounds__(BS) void k_replicas(const Rep *__restrict__ reps, c
   const bool allpairs = R.S == 0;
   const int ncell = allpairs ? 0 : R.nc[0] * R.nc[1] * R.nc[2];
   const int chunk = (ncell + BS - 1) / BS;
+  const int G = atom_lanes(n);
   double pe = 0.0, ke = 0.0, vir = 0.0;
 
+  // the atom's cell for the next scatter: its rank among the cell's atoms so far
+  auto bin = [&](int g, float px, float py, float pz) {
+    if (allpairs) return;
+    const int cell = (cell_coord(pz, R.halfL[2], R.cinv[2], R.nc[2]) * R.nc[1] +
+                      cell_coord(py, R.halfL[1], R.cinv[1], R.nc[1])) * R.nc[0] +
+                     cell_coord(px, R.halfL[0], R.cinv[0], R.nc[0]);
+    const int sh = 16 * (cell & 1);
+    const unsigned r = (atomicAdd(&cnt[cell >> 1], 1u << sh) >> sh) & 0xffffu;
+    key[g] = (int)((unsigned)cell | (r << 16));
+  };
+  // opening half kick, drift and wrap of one atom
+  auto kick_drift = [&](int g, float ux, float uy, float uz, float px, float py, float pz) {
+    vx[g] = ux; vy[g] = uy; vz[g] = uz;
+    px = wrap_centred(fmaf(dt, ux, px), R.L[0]);
+    py = wrap_centred(fmaf(dt, uy, py), R.L[1]);
+    pz = wrap_centred(fmaf(dt, uz, pz), R.L[2]);
+    x[g] = px; y[g] = py; z[g] = pz;
+    bin(g, px, py, pz);
+  };
+
+  for (int k = t; k < (ncell + 1) / 2; k += BS) cnt[k] = 0u;
+  __syncthreads();
+  for (int i = t; i < n; i += BS) {
+    const int g = off + i;
+    if (first_force) bin(g, x[g], y[g], z[g]);
+    else kick_drift(g, fmaf(c, fx[g], vx[g]), fmaf(c, fy[g], vy[g]), fmaf(c, fz[g], vz[g]), x[g], y[g], z[g]);
+  }
+  __syncthreads();
   for (int step = first_force ? 0 : 1; step <= nsteps; ++step) {
     const bool integrate = step > 0;
     const bool last = step == nsteps;
-    // ---- A: kick-drift, cell counts
-    for (int k = t; k < ncell; k += BS) cnt[k] = 0;
-    __syncthreads();
-    for (int i = t; i < n; i += BS) {
-      const int g = off + i;
-      float px = x[g], py = y[g], pz = z[g];
-      if (integrate) {
-        const float ux = fmaf(c, fx[g], vx[g]), uy = fmaf(c, fy[g], vy[g]), uz = fmaf(c, fz[g], vz[g]);
-        vx[g] = ux; vy[g] = uy; vz[g] = uz;
-        px = wrap_centred(fmaf(dt, ux, px), R.L[0]);
-        py = wrap_centred(fmaf(dt, uy, py), R.L[1]);
-        pz = wrap_centred(fmaf(dt, uz, pz), R.L[2]);
-        x[g] = px; y[g] = py; z[g] = pz;
-      }
-      if (allpairs) {
-        spos[i] = make_float4(px, py, pz, __int_as_float(i));
-      } else {
-        const int cell = (cell_coord(pz, R.halfL[2], R.cinv[2], R.nc[2]) * R.nc[1] +
-                          cell_coord(py, R.halfL[1], R.cinv[1], R.nc[1])) * R.nc[0] +
-                         cell_coord(px, R.halfL[0], R.cinv[0], R.nc[0]);
-        const int r = atomicAdd(&cnt[cell], 1);
-        key[g] = cell | (r << 16);
-      }
-    }
-    __syncthreads();
     if (!allpairs) {
       // ---- B: exclusive scan of the counts (contiguous chunk per thread, wave scans)
       const int k0 = min(t * chunk, ncell), k1 = min(k0 + chunk, ncell);
+      auto count = [&](int k) { return (int)((cnt[k >> 1] >> (16 * (k & 1))) & 0xffffu); };
       int sum = 0;
-      for (int k = k0; k < k1; ++k) sum += cnt[k];
+      for (int k = k0; k < k1; ++k) sum += count(k);
       int v = sum;
 #pragma unroll
       for (int o = 1; o < WAVE; o <<= 1) {
@@ -139,17 +232,17 @@ __global__ __launch_bounds__(BS) void k_replicas(const Rep *__restrict__ reps, c
       int base = v - sum;
       for (int w = 0; w < wave; ++w) base += wsum[w];
       for (int k = k0; k < k1; ++k) {
-        const int ck = cnt[k];
         cst[k] = (unsigned short)base;
-        base += ck;
+        base += count(k);
       }
       if (t == 0) cst[ncell] = (unsigned short)n;
       __syncthreads();
-      // ---- C: scatter into cell order (overwrites the counts)
+      // ---- C: scatter into cell order; the counts are cleared for E
+      for (int k = t; k < (ncell + 1) / 2; k += BS) cnt[k] = 0u;
       for (int i = t; i < n; i += BS) {
         const int g = off + i;
-        const int kk = key[g];
-        const int slot = cst[kk & 0xffff] + (kk >> 16);
+        const unsigned kk = (unsigned)key[g];
+        const int slot = cst[kk & 0xffffu] + (int)(kk >> 16);
         spos[slot] = make_float4(x[g], y[g], z[g], __int_as_float(i));
       }
       __syncthreads();
@@ -167,75 +260,40 @@ __global__ __launch_bounds__(BS) void k_replicas(const Rep *__restrict__ reps, c
           spos[j + 1] = p;
         }
       }
-      __syncthreads();
+    } else {
+      for (int i = t; i < n; i += BS) spos[i] = make_float4(x[off + i], y[off + i], z[off + i], __int_as_float(i));
     }
-    // ---- E: forces and the closing kick
+    __syncthreads();
+    // ---- E: forces, the closing kick, and the next step's kick-drift and cell count
     const bool acc = last && energy;
-    for (int s = t; s < n; s += BS) {
+    for (int q = t; q < n * G; q += BS) {
+      const int s = q / G, sub = q - s * G;
       const float4 p = spos[s];
       float ax = 0.f, ay = 0.f, az = 0.f, e = 0.f, w = 0.f;
-      if (allpairs) {
-        for (int j = 0; j < n; ++j) {
-          const float4 q = spos[j];
-          const float dx = mic_fast(p.x - q.x, R.halfL[0], R.L[0]);
-          const float dy = mic_fast(p.y - q.y, R.halfL[1], R.L[1]);
-          const float dz = mic_fast(p.z - q.z, R.halfL[2], R.L[2]);
-          const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-          float f, u;
-          lj_terms(R, j == s ? 0.f : r2, f, u);
-          ax = fmaf(f, dx, ax); ay = fmaf(f, dy, ay); az = fmaf(f, dz, az);
-          e += u;
-          w = fmaf(f, r2, w);
-        }
-      } else {
-        const int cx = cell_coord(p.x, R.halfL[0], R.cinv[0], R.nc[0]);
-        const int cy = cell_coord(p.y, R.halfL[1], R.cinv[1], R.nc[1]);
-        const int cz = cell_coord(p.z, R.halfL[2], R.cinv[2], R.nc[2]);
-        for (int dz3 = -R.S; dz3 <= R.S; ++dz3) {
-          int zz = cz + dz3;
-          zz += zz < 0 ? R.nc[2] : 0;
-          zz -= zz >= R.nc[2] ? R.nc[2] : 0;
-          for (int dy3 = -R.S; dy3 <= R.S; ++dy3) {
-            int yy = cy + dy3;
-            yy += yy < 0 ? R.nc[1] : 0;
-            yy -= yy >= R.nc[1] ? R.nc[1] : 0;
-            const int row = (zz * R.nc[1] + yy) * R.nc[0];
-            for (int dx3 = -R.S; dx3 <= R.S; ++dx3) {
-              int xx = cx + dx3;
-              xx += xx < 0 ? R.nc[0] : 0;
-              xx -= xx >= R.nc[0] ? R.nc[0] : 0;
-              const int cell = row + xx;
-              const int b = cst[cell], en = cst[cell + 1];
-              for (int j = b; j < en; ++j) {
-                const float4 q = spos[j];
-                const float dx = mic_fast(p.x - q.x, R.halfL[0], R.L[0]);
-                const float dy = mic_fast(p.y - q.y, R.halfL[1], R.L[1]);
-                const float dz = mic_fast(p.z - q.z, R.halfL[2], R.L[2]);
-                const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-                float f, u;
-                lj_terms(R, j == s ? 0.f : r2, f, u);
-                ax = fmaf(f, dx, ax); ay = fmaf(f, dy, ay); az = fmaf(f, dz, az);
-                e += u;
-                w = fmaf(f, r2, w);
-              }
-            }
-          }
-        }
-      }
-      const int g = off + __float_as_int(p.w);
-      fx[g] = ax; fy[g] = ay; fz[g] = az;
-      float ux = vx[g], uy = vy[g], uz = vz[g];
-      if (integrate) {
-        ux = fmaf(c, ax, ux); uy = fmaf(c, ay, uy); uz = fmaf(c, az, uz);
-        vx[g] = ux; vy[g] = uy; vz[g] = uz;
+      if (acc) atom_forces<true>(R, spos, cst, n, p, s, sub, G, ax, ay, az, e, w);
+      else atom_forces<false>(R, spos, cst, n, p, s, sub, G, ax, ay, az, e, w);
+      for (int o = G >> 1; o >= 1; o >>= 1) {  // n G and the stride are multiples of G: whole groups
+        ax += __shfl_xor(ax, o, WAVE);
+        ay += __shfl_xor(ay, o, WAVE);
+        az += __shfl_xor(az, o, WAVE);
       }
       if (acc) {
         pe += 0.5 * (double)e;
         vir += 0.5 * (double)w;
-        ke += 0.5 * (double)mass * ((double)ux * ux + (double)uy * uy + (double)uz * uz);
+      }
+      if (sub != 0) continue;
+      const int g = off + __float_as_int(p.w);
+      float ux = vx[g], uy = vy[g], uz = vz[g];
+      if (integrate) { ux = fmaf(c, ax, ux); uy = fmaf(c, ay, uy); uz = fmaf(c, az, uz); }
+      if (last) {
+        fx[g] = ax; fy[g] = ay; fz[g] = az;
+        if (integrate) { vx[g] = ux; vy[g] = uy; vz[g] = uz; }
+        if (acc) ke += 0.5 * (double)mass * ((double)ux * ux + (double)uy * uy + (double)uz * uz);
+      } else {
+        kick_drift(g, fmaf(c, ax, ux), fmaf(c, ay, uy), fmaf(c, az, uz), p.x, p.y, p.z);
       }
     }
-    __syncthreads();  // spos / cnt are rewritten by the next step
+    __syncthreads();  // spos is rewritten by the next step; its x, key and counts are complete
   }
   if (energy) {
     const double a = block_sum<BS>(pe, red);
@@ -258,16 +316,18 @@ struct pdx_rep_s {
   std::vector<pdx_replica_spec> specs;
   std::vector<Rep> host;
   std::vector<int64_t> offsets;
-  int nrep = 0, nmax = 0, ncmax = 0, block = 512, stencil = 1, nallpairs = 0;
+  int nrep = 0, nmax = 0, ncmax = 0, block = 1024, stencil = 0, nallpairs = 0;
   int64_t total = 0;
-  size_t reg0 = 0, reg1 = 0, lds = 0;
+  size_t reg0 = 0, reg1 = 0, reg2 = 0, lds = 0;
+
   DevBuf<Rep> reps;
   DevBuf<int32_t> order, key;
 };
 
 namespace {
 
-// Cell tables for stencil half-width S (1 or 2): cells of side >= rc / S, at least 2S + 1 a
+// Cell tables for stencil half-width S (1 or 2; 0: per replica, 2 where its finer cells fit the
+// table): cells of side >= rc / S, at least 2S + 1 a
 // side (else S = 1, else all pairs), at most NCMAX cells (the widest dimension is coarsened).
 int layout(pdx_rep_t r, int S) {
   r->host.resize(r->nrep);
@@ -294,6 +354,17 @@ int layout(pdx_rep_t r, int S) {
       R.halfL[d] = (float)(0.5 * sp.box[d]);
     }
     int s = S;
+    if (S == 0) {
+      // halved cells cut the candidates of a sphere of rc (8192 LJ atoms: 430 -> about 150 with the
+      // rows cut to the sphere); where they would have to be coarsened, whole cells are walked
+      // (boxes with fewer than three whole cells a side take all pairs)
+      double fine = 1.0, least = sp.box[0];
+      for (int d = 0; d < 3; ++d) {
+        fine *= std::floor(sp.box[d] * 2 / rc);
+        least = std::min(least, sp.box[d]);
+      }
+      s = fine <= (double)NCMAX && least >= 3.0 * rc ? 2 : 1;
+    }
     int nc[3];
     for (; s >= 1; --s) {
       bool ok = true;
@@ -319,15 +390,18 @@ int layout(pdx_rep_t r, int S) {
       for (int d = 0; d < 3; ++d) {
         R.nc[d] = nc[d];
         R.cinv[d] = (float)(nc[d] / sp.box[d]);
+        R.cw[d] = (float)(sp.box[d] / nc[d]);
+        R.slack = std::max(R.slack, (float)(2e-6 * sp.box[d]));
       }
       r->ncmax = std::max(r->ncmax, nc[0] * nc[1] * nc[2]);
     }
     r->nmax = std::max(r->nmax, R.n);
     r->host[k] = R;
   }
-  r->reg0 = align16(std::max<size_t>(16 * (size_t)r->nmax, 4 * (size_t)r->ncmax));
+  r->reg0 = 16 * (size_t)r->nmax;
   r->reg1 = align16(2 * ((size_t)r->ncmax + 1));
-  r->lds = r->reg0 + r->reg1 + 128 + RED_BYTES;
+  r->reg2 = align16(2 * ((size_t)r->ncmax + 1));
+  r->lds = r->reg0 + r->reg1 + r->reg2 + 128 + RED_BYTES;
   if (r->lds > 160 * 1024) return fail(PDX_ERR_ARGUMENT, "replica tables exceed the 160 KiB of LDS");
   if (hipMemcpy(r->reps.p, r->host.data(), sizeof(Rep) * r->nrep, hipMemcpyHostToDevice) != hipSuccess)
     return fail(PDX_ERR_DEVICE, "replica table upload failed");
@@ -359,7 +433,8 @@ int launch(pdx_rep_t r, float *x, float *y, float *z, float *vx, float *vy, floa
     attr = true;
   }
   hipLaunchKernelGGL(k_replicas<BS>, dim3(r->nrep), dim3(BS), r->lds, st, r->reps.p, r->order.p, x, y, z, vx, vy,
-                     vz, fx, fy, fz, r->key.p, c, dt, mass, nsteps, first, energy, (int)r->reg0, (int)r->reg1, out);
+                     vz, fx, fy, fz, r->key.p, c, dt, mass, nsteps, first, energy, (int)r->reg0, (int)r->reg1,
+                     (int)r->reg2, out);
   PDX_LAUNCH_CHECK();
   return PDX_OK;
 }
@@ -371,10 +446,10 @@ extern "C" int pdx_replicas_create(int32_t nrep, const pdx_replica_spec *specs, 
   if (!out || !specs) return fail(PDX_ERR_ARGUMENT, "null argument");
   *out = nullptr;
   if (nrep < 1) return fail(PDX_ERR_ARGUMENT, "at least one replica is required");
-  if (block == 0) block = 512;
+  // 1024 threads: the coordinates of the largest replicas leave room for one workgroup per CU
+  if (block == 0) block = 1024;
   if (block != 256 && block != 512 && block != 1024) return fail(PDX_ERR_ARGUMENT, "block must be 256, 512 or 1024");
-  if (stencil == 0) stencil = 1;
-  if (stencil != 1 && stencil != 2) return fail(PDX_ERR_ARGUMENT, "stencil must be 1 or 2");
+  if (stencil != 0 && stencil != 1 && stencil != 2) return fail(PDX_ERR_ARGUMENT, "stencil must be 1 or 2");
   int64_t total = 0;
   for (int k = 0; k < nrep; ++k) {
     const pdx_replica_spec &s = specs[k];

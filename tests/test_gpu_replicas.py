@@ -165,3 +165,33 @@ def test_energy_conservation(cuda):
               flush=True)
         assert abs(E0 - (pa + ka)) < 1e-5 * abs(pa + ka) + 1e-3
         assert abs(drift - ref) < 1e-3 + 0.1 * abs(ref), (k, drift, ref)
+
+
+@pytest.mark.parametrize("n", [3, 512, 513, 1024, 1025, 8192])
+@pytest.mark.parametrize("model,aspect", [("lj", (1.0, 1.0, 1.0)), ("lj", (0.8, 1.0, 1.25)), ("wca", (1.3, 1.0, 0.77))])
+def test_forces_at_the_size_steps(cuda, n, model, aspect):
+    """The sizes where the lanes per atom change, the largest replica and a nearly empty box, cubic
+    and not, with the cells chosen by the library: forces and energies against the FP64 sums."""
+    rng = np.random.default_rng(n)
+    side = max((n / 0.8) ** (1.0 / 3.0), 8.0)
+    box = tuple(side * a for a in aspect)
+    m = int(np.ceil(n ** (1.0 / 3.0)))
+    g = np.stack(np.meshgrid(*(np.arange(m),) * 3, indexing="ij"), -1).reshape(-1, 3)[rng.permutation(m ** 3)[:n]]
+    L = np.array(box)
+    # on a lattice of m sites a side, jittered by 8 % of the spacing; some atoms on the faces
+    X = ((g + 0.08 * rng.standard_normal(g.shape)) / m - 0.5) * L
+    X = (X - L * np.floor(X / L + 0.5)).astype(np.float32)
+    L32 = L.astype(np.float32)
+    X = np.where(X >= L32 / 2, -L32 / 2, X)
+    bd = dict(x=X[:, 0], y=X[:, 1], z=X[:, 2], vx=np.zeros(n), vy=np.zeros(n), vz=np.zeros(n))
+    rb = pdx.ReplicaBatch([{"model": model, "n": n, "box": box, "cutoff": 2.5, "shift": False}])
+    st = replicas.device_state(bd)
+    out = rb.forces(st).cpu().numpy()[0]
+    h = _host(st, 0, rb.offsets)
+    d = oracle.pair_direct(h["x"], h["y"], h["z"], box, kind=model, cutoff=2.5)
+    F = np.stack([h["fx"], h["fy"], h["fz"]], 1)
+    # the FP32 bounds of the other force tests (2e-5 of the forces, 1e-5 of the energies)
+    assert np.linalg.norm(F - d["F"]) <= 2e-5 * np.linalg.norm(d["F"])
+    assert abs(out[0] - d["energy"].sum()) <= 1e-5 * max(np.abs(d["energy"]).sum(), 1e-30)
+    assert abs(out[2] - d["virial"][:, :3].sum()) <= 1e-5 * max(np.abs(d["virial"]).sum(), 1e-30)
+    assert out[3] == n
