@@ -278,7 +278,8 @@ __global__ __launch_bounds__(SUM_THREADS) void k_sum_partials(const double *__re
 struct pdx_nl_s {
   int32_t N = 0, cap = 0, nx = 1, ny = 1, nz = 1, ncell = 1;
   int32_t interval = 20;
-  int32_t row_lanes = 1;  // lanes per particle of the row build
+  int32_t row_lanes = 1;  // lanes per particle of k_rows
+  bool row_lanes_given = false;  // a caller's choice: k_rows builds the rows
   bool allpairs = false, diagnostics = false;
   int dim = 3;  // 2: no z coordinates (z = 0), box[2] is the list's own z extent of three radii
   double box[3] = {0, 0, 0};
@@ -294,8 +295,8 @@ struct pdx_nl_s {
   pdx::DevBuf<float4> sortedq;  // N, cell order, current (x, y, z, q): the cell traversal's copy
   pdx::DevBuf<float> disp_partial;  // ndisp per-block maxima of the last check
   int32_t ndisp = 0;
-  pdx::DevBuf<int32_t> cap_partial;
-  pdx::DevBuf<int64_t> stat_partial;  // 2 per block: candidates, accepted
+  pdx::DevBuf<int32_t> row_max;       // largest row of the build under way
+  pdx::DevBuf<int64_t> stat_partial;  // 2 per row block: candidates, accepted
   pdx::DevBuf<int32_t> scan_block;    // per-1024-cell block totals
   pdx::DevBuf<int64_t> candidates;    // N (diagnostics)
   // cell snapshot for a spread that runs beside the rebuild: offsets and ids of the last

@@ -12,12 +12,12 @@
 //   k_scatter      particle_ids_sorted (1-based)
 //   k_sort_cells   ascending id inside each cell (rows and traversal become reproducible),
 //                  and the cell-ordered packed positions read by the row kernel
-//   k_rows         27-cell stencil, r^2 <= rlist^2, slot-major rows t*N + i, 1-based ids
-//   k_commit       per-block max row length and statistics
-//   k_commit_final max row length vs cap, state words (one wave)
-//   k_copy_refs    reference positions of the successful build
+//   k_rows_masks   (or k_rows / k_rows_cells / k_rows_allpairs) 27-cell stencil, r^2 <= rlist^2,
+//                  slot-major rows t*N + i, 1-based ids; per-block max row length and statistics
+//   k_commit_refs  max row length vs cap, state words; reference positions of a successful build
 #include "pdx_internal.hpp"
 
+#include <algorithm>
 #include <cmath>
 #include <cstdlib>
 
@@ -54,7 +54,7 @@ __global__ __launch_bounds__(TPB) void k_decide(int N, float *__restrict__ x,
                                                  float *__restrict__ z,
                                                  const float *__restrict__ q,
                                                  const float *__restrict__ rref, float4 *packed,
-                                                 int32_t *cell_counts, int ncell, int allpairs,
+                                                 int32_t *cell_counts, int32_t *row_max, int ncell, int allpairs,
                                                  const float *geom, const int64_t *state,
                                                  float *partial, const int32_t *__restrict__ offsets,
                                                  const int32_t *__restrict__ ids, int32_t *snap_offsets,
@@ -105,7 +105,8 @@ __global__ __launch_bounds__(TPB) void k_decide(int N, float *__restrict__ x,
     }
     packed[i] = make_float4(c[0], c[1], c[2], q ? q[i] : 0.0f);
   }
-  // histogram storage is scratch of the next rebuild: clear it here (one launch fewer)
+  // histogram and largest row are scratch of the next rebuild: cleared here (one launch fewer)
+  if (i == 0) *row_max = 0;
   if (!allpairs)
     for (int c = i; c < ncell; c += gridDim.x * TPB) cell_counts[c] = 0;
 
@@ -192,18 +193,6 @@ __global__ __launch_bounds__(TPB) void k_bin(int N, const float4 *__restrict__ p
   const int c = (cz * ny + cy) * nx + cx;
   cell_of_particle[i] = c;
   cell_rank[i] = atomicAdd(&cell_counts[c], 1);
-}
-
-// Reference positions of a successful build (skipped when the commit latched an error).
-__global__ __launch_bounds__(TPB) void k_copy_refs(int N, const float4 *__restrict__ packed,
-                                                    float *rref, const int64_t *state) {
-  if (!rebuild_requested(state)) return;
-  const int i = blockIdx.x * TPB + threadIdx.x;
-  if (i >= N) return;
-  const float4 p = packed[i];
-  rref[i] = p.x;
-  rref[(size_t)N + i] = p.y;
-  rref[(size_t)2 * N + i] = p.z;
 }
 
 // Cell offsets in one launch for grids of up to 16384 cells: 1024 threads, a contiguous run of
@@ -301,9 +290,9 @@ __global__ __launch_bounds__(TPB) void k_scan_finish(int ncell, int N, int32_t *
   if (c == ncell) offsets[ncell] = N + 1;
 }
 
-__global__ __launch_bounds__(TPB) void k_scatter(int N, const int32_t *cell_of_particle,
-                                                  const int32_t *cell_rank,
-                                                  const int32_t *offsets, int32_t *ids_sorted,
+__global__ __launch_bounds__(TPB) void k_scatter(int N, const int32_t *__restrict__ cell_of_particle,
+                                                  const int32_t *__restrict__ cell_rank,
+                                                  const int32_t *__restrict__ offsets, int32_t *ids_sorted,
                                                   const int64_t *state) {
   if (!rebuild_requested(state)) return;
   const int i = blockIdx.x * TPB + threadIdx.x;
@@ -373,6 +362,28 @@ __global__ __launch_bounds__(WAVE) void k_sort_cells(int ncell, const int32_t *o
 // consecutive particles is one contiguous store; written straight from the search, the slots of
 // a wave's particles advance at different rates and the 4-byte stores land in partially filled
 // lines (measured: 8.6x the row bytes at 486 400 ions, 2.0x staged). Same rows either way.
+// Commit data of a block's rows (_device_capacity_partial_kernel!, DeviceNeighborCUDA.jl:291-310): the
+// largest row into one word, candidates and accepted entries per block; called by every thread.
+__device__ __forceinline__ void row_partials(int longest, long long tested, long long accepted, int32_t *row_max,
+                                             int64_t *stat_partial) {
+  __shared__ int smax[TPB / WAVE];
+  __shared__ long long ssum[2][TPB / WAVE];
+  longest = wave_max(longest);
+  for (int off = 32; off >= 1; off >>= 1) {
+    tested += __shfl_xor(tested, off, WAVE);
+    accepted += __shfl_xor(accepted, off, WAVE);
+  }
+  const int w = threadIdx.x / WAVE, nw = blockDim.x / WAVE;
+  if ((threadIdx.x & (WAVE - 1)) == 0) { smax[w] = longest; ssum[0][w] = tested; ssum[1][w] = accepted; }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int k = 1; k < nw; ++k) { longest = max(longest, smax[k]); tested += ssum[0][k]; accepted += ssum[1][k]; }
+    atomicMax(row_max, longest);
+    stat_partial[2 * blockIdx.x] = tested;
+    stat_partial[2 * blockIdx.x + 1] = accepted;
+  }
+}
+
 constexpr size_t ROW_STAGE_BYTES = 65536;
 template <int G, bool STAGE>
 __global__ __launch_bounds__(TPB) void k_rows(int N, int cap, int nx, int ny, int nz,
@@ -380,8 +391,8 @@ __global__ __launch_bounds__(TPB) void k_rows(int N, int cap, int nx, int ny, in
                                                const int32_t *__restrict__ offsets,
                                                const int32_t *__restrict__ cell_of_particle,
                                                const float *geom, float rl2, int32_t *nbr,
-                                               int32_t *counts, int64_t *candidates,
-                                               const int64_t *state) {
+                                               int32_t *counts, int64_t *candidates, int32_t *row_max,
+                                               int64_t *stat_partial, const int64_t *state) {
   constexpr int PB = TPB / G;  // particles per workgroup
   extern __shared__ int32_t srow[];  // STAGE: [cap][PB]
   __shared__ int sfound[PB], sid[PB];
@@ -471,6 +482,8 @@ __global__ __launch_bounds__(TPB) void k_rows(int N, int cap, int nx, int ny, in
     counts[i] = found;
     if (candidates) candidates[i] = tested;
   }
+  const bool own = active && lg == 0;
+  row_partials(own ? found : 0, own ? tested : 0, own ? found : 0, row_max, stat_partial);
 }
 
 // Rows from LDS-staged candidates: one workgroup per cell. Wave 0 lists the cell's 27 stencil cells
@@ -485,11 +498,14 @@ __global__ __launch_bounds__(TPB) void k_rows_cells(int N, int cap, int ncell, i
                                                     const float4 *__restrict__ sorted,
                                                     const int32_t *__restrict__ offsets, const float *geom,
                                                     float rl2, int32_t *nbr, int32_t *counts,
-                                                    int64_t *candidates, const int64_t *state) {
+                                                    int64_t *candidates, int32_t *row_max,
+                                                    int64_t *stat_partial, const int64_t *state) {
   constexpr int PB = TPB / G;  // particles per pass
   __shared__ float4 cand[RC_CHUNK];
   __shared__ int cstart[27], cpre[28];
   if (!rebuild_requested(state)) return;  // uniform over the grid
+  int longest = 0;
+  long long all_tested = 0, all_found = 0;
   for (int c = blockIdx.x; c < ncell; c += gridDim.x) {  // grid-stride over the cells
     const int p0 = offsets[c] - 1, np = offsets[c + 1] - offsets[c];
     if (np <= 0) continue;  // uniform over the workgroup
@@ -580,9 +596,173 @@ __global__ __launch_bounds__(TPB) void k_rows_cells(int N, int cap, int ncell, i
       if (active && lg == 0) {
         counts[i] = found;
         if (candidates) candidates[i] = tested;
+        longest = max(longest, found);
+        all_tested += tested;
+        all_found += found;
       }
     }
   }
+  row_partials(longest, all_tested, all_found, row_max, stat_partial);
+}
+
+// ---- the default build of many well-filled cells: one workgroup per cell, lanes = candidates,
+// particles one after the other in scalar registers (four waves, a chunk of 64 candidates each in
+// turn). A distance test of 64 candidates is then seven vector instructions (three more per
+// dimension where the stencil crosses the seam), its ballot goes into lane p of a register pair (particle p of the cell), and the cell's tests end as bit
+// masks in LDS. The rows are written in a second pass with lanes = particles, each wave a quarter of
+// the masks from the slot its earlier ones add up to: every lane takes its next set bit, so a store
+// writes neighbouring slots of the cell's rows, lines that fill up within a few steps where the
+// cell's particles are contiguous in storage (spatial order). Candidates are numbered in stencil
+// order (z, y, x cells, then the cells' order), so rows are k_rows' rows.
+// Bound by vector issue in both passes (about 9 instructions per 64 tests and 12 per step of the row
+// writes). k_rows spends 38 on 64 tests (per-lane image, ballots, predicated 4-byte stores that each
+// touch their own line). Whole rebuilds with it at its best lane count and with this kernel: 326 and
+// 264 us (256 000 LJ atoms, 21 a cell), 1 224 and 1 020 us (486 400 ions, 61 a cell).
+// v_writelane_b32 (this compiler has the intrinsic but no builtin for it): old with lane `lane` = value,
+// both uniform.
+extern "C" __device__ __attribute__((const)) int pdx_writelane(int value, int lane, int old) __asm("llvm.amdgcn.writelane.i32");
+constexpr int RM_CHUNKS = 28;  // candidate chunks of 64 per pass (21 KiB of LDS: seven workgroups per CU)
+constexpr int RM_WAVES = TPB / WAVE;
+__global__ __launch_bounds__(TPB) void k_rows_masks(int N, int cap, int ncell, int nx, int ny, int nz,
+                                                     const float4 *__restrict__ sorted,
+                                                     const int32_t *__restrict__ offsets,
+                                                     const float *__restrict__ geom, float rl2,
+                                                     int32_t *__restrict__ nbr, int32_t *__restrict__ counts,
+                                                     int64_t *candidates, int32_t *row_max, int64_t *stat_partial,
+                                                     const int64_t *state) {
+  __shared__ uint2 mask[RM_CHUNKS][WAVE];
+  __shared__ int32_t cid[RM_CHUNKS * WAVE];
+  __shared__ int cstart[27], cpre[28], ends[WAVE];
+  if (!rebuild_requested(state)) return;  // uniform over the grid
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x / WAVE);
+  const float Lx = geom[0], Ly = geom[1], Lz = geom[2];
+  const float hx = 0.5f * Lx, hy = 0.5f * Ly, hz = 0.5f * Lz;
+  int longest = 0;
+  long long all_tested = 0, all_found = 0;
+  for (int c = blockIdx.x; c < ncell; c += gridDim.x) {
+    const int p0 = offsets[c] - 1, np = offsets[c + 1] - 1 - p0;  // uniform
+    if (np <= 0) continue;
+    const int cx = c % nx, cy = (c / nx) % ny, cz = c / (nx * ny);
+    __syncthreads();  // the previous cell's LDS is no longer read
+    if (wv == 0) {
+      int cnt = 0;
+      if (lane < 27) {
+        int cz2 = cz + lane / 9 - 1; cz2 -= (cz2 >= nz) ? nz : 0; cz2 += (cz2 < 0) ? nz : 0;
+        int cy2 = cy + (lane / 3) % 3 - 1; cy2 -= (cy2 >= ny) ? ny : 0; cy2 += (cy2 < 0) ? ny : 0;
+        int cx2 = cx + lane % 3 - 1; cx2 -= (cx2 >= nx) ? nx : 0; cx2 += (cx2 < 0) ? nx : 0;
+        const int cc = (cz2 * ny + cy2) * nx + cx2;
+        cstart[lane] = offsets[cc] - 1;
+        cnt = offsets[cc + 1] - offsets[cc];
+      }
+#pragma unroll
+      for (int d = 1; d < WAVE; d <<= 1) {
+        const int u = __shfl_up(cnt, d, WAVE);
+        if (lane >= d) cnt += u;
+      }
+      if (lane < 27) cpre[lane + 1] = cnt;
+      if (lane == 0) cpre[0] = 0;
+    }
+    __syncthreads();
+    const int total = __builtin_amdgcn_readfirstlane(cpre[27]);
+    const int self0 = __builtin_amdgcn_readfirstlane(cpre[13]);  // the home cell's first candidate
+    // no cell of the stencil lies across the seam, and two cells apart is less than half the box
+    const bool plain = cx > 0 && cx < nx - 1 && cy > 0 && cy < ny - 1 && cz > 0 && cz < nz - 1 && nx > 4 && ny > 4 &&
+                       nz > 4;
+    for (int pg = 0; pg < np; pg += WAVE) {
+      const int ng = min(WAVE, np - pg);
+      const float4 *home = sorted + p0 + pg;
+      const int i = lane < ng ? __float_as_int(home[lane].w) : 0;
+      int found = 0;
+      for (int ch0 = 0; ch0 < total; ch0 += RM_CHUNKS * WAVE) {
+        const int nch = min(RM_CHUNKS, (total - ch0 + WAVE - 1) / WAVE);
+        for (int cc = wv; cc < nch; cc += RM_WAVES) {
+          const int g = ch0 + cc * WAVE + lane;
+          int sc = 0;
+#pragma unroll
+          for (int h = 16; h >= 1; h >>= 1)
+            if (sc + h < 27 && cpre[sc + h] <= g) sc += h;
+          // lanes past the last candidate sit too far from everything to be accepted
+          float4 q = make_float4(1e30f, 0.f, 0.f, 0.f);
+          if (g < total) q = sorted[cstart[sc] + (g - cpre[sc])];
+          cid[cc * WAVE + lane] = __float_as_int(q.w) + 1;
+          int mlo = 0, mhi = 0;
+          auto test = [&](int p, const float4 &pi, auto image) {
+            float dx = q.x - pi.x, dy = q.y - pi.y, dz = q.z - pi.z;
+            image(dx, dy, dz);
+            const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+            const unsigned long long m = __ballot(r2 <= rl2);
+            mlo = pdx_writelane((int)(unsigned)m, p, mlo);
+            mhi = pdx_writelane((int)(unsigned)(m >> 32), p, mhi);
+          };
+          // four particles' scalar loads in flight (lanes past ng - 1 of the masks are not read)
+          auto tests = [&](auto image) {
+            for (int p = 0; p < ng; p += 4) {
+              float4 pi[4];
+#pragma unroll
+              for (int u = 0; u < 4; ++u) pi[u] = home[min(p + u, ng - 1)];
+#pragma unroll
+              for (int u = 0; u < 4; ++u) test(p + u, pi[u], image);
+            }
+          };
+          // k_bin puts a particle at the very face +L/2 into cell 0: next to it, in cell 1, its
+          // distance still needs the image
+          const bool face = g < total && ((cx == 1 && q.x > 0.5f * hx) || (cy == 1 && q.y > 0.5f * hy) ||
+                                          (cz == 1 && q.z > 0.5f * hz));
+          if (plain && __ballot(face) == 0) {
+            tests([](float &, float &, float &) {});
+          } else {
+            tests([&](float &dx, float &dy, float &dz) {
+              dx = mic_fast(dx, hx, Lx);
+              dy = mic_fast(dy, hy, Ly);
+              dz = mic_fast(dz, hz, Lz);
+            });
+          }
+          // the particle itself is among the home cell's candidates
+          const int b = self0 + pg + lane - ch0 - cc * WAVE;
+          if (b >= 0 && b < 32) mlo &= (int)~(1u << b);
+          if (b >= 32 && b < WAVE) mhi &= (int)~(1u << (b - 32));
+          mask[cc][lane] = make_uint2((unsigned)mlo, (unsigned)mhi);
+        }
+        __syncthreads();
+        auto word = [&](int k) {
+          const uint2 m = mask[k][lane];
+          return lane < ng ? ((unsigned long long)m.y << 32) | m.x : 0ull;
+        };
+        const int w0 = nch * wv / RM_WAVES, w1 = nch * (wv + 1) / RM_WAVES;
+        for (int k = 0; k < w0; ++k) found += (int)__popcll(word(k));
+        int w = w0;
+        unsigned long long m = w0 < w1 ? word(w0) : 0ull, nextm = w0 + 1 < w1 ? word(w0 + 1) : 0ull;
+        int32_t *out = nbr + (size_t)found * N + i;
+        while (__ballot(m != 0ull || w < w1 - 1) != 0) {
+          if (m == 0ull && w < w1 - 1) {
+            ++w;
+            m = nextm;
+            nextm = w + 1 < w1 ? word(w + 1) : 0ull;
+          }
+          if (m != 0ull) {
+            const int b = __ffsll((long long)m) - 1;
+            m &= m - 1ull;
+            const int j = cid[w * WAVE + b];
+            if (found < cap) *out = j;
+            out += N;
+            ++found;
+          }
+        }
+        if (wv == RM_WAVES - 1) ends[lane] = found;
+        __syncthreads();
+        found = ends[lane];
+      }
+      if (wv == 0 && lane < ng) {
+        counts[i] = found;
+        if (candidates) candidates[i] = total - 1;
+        longest = max(longest, found);
+        all_tested += total - 1;
+        all_found += found;
+      }
+    }
+  }
+  row_partials(longest, all_tested, all_found, row_max, stat_partial);
 }
 
 // All-pairs rows for small boxes, one image (_kernel_neighbors_allpairs!, DenseNeighborCUDA.jl:128-151).
@@ -590,76 +770,66 @@ __global__ __launch_bounds__(TPB) void k_rows_allpairs(int N, int cap,
                                                         const float4 *__restrict__ packed,
                                                         const float *geom, float rl2,
                                                         int32_t *nbr, int32_t *counts,
-                                                        int64_t *candidates,
-                                                        const int64_t *state) {
+                                                        int64_t *candidates, int32_t *row_max,
+                                                        int64_t *stat_partial, const int64_t *state) {
   if (!rebuild_requested(state)) return;
   const int i = blockIdx.x * TPB + threadIdx.x;
-  if (i >= N) return;
-  const float Lx = geom[0], Ly = geom[1], Lz = geom[2];
-  const float4 pi = packed[i];
+  const bool active = i < N;
   int found = 0;
-  for (int j = 0; j < N; ++j) {
-    if (j == i) continue;
-    const float4 pj = packed[j];
-    // dimension order of the reference's loop: r2 = muladd(dd, dd, r2) for d = 1..D
-    float r2 = 0.0f;
-    float dd = mic_fast(pj.x - pi.x, 0.5f * Lx, Lx); r2 = fmaf(dd, dd, r2);
-    dd = mic_fast(pj.y - pi.y, 0.5f * Ly, Ly); r2 = fmaf(dd, dd, r2);
-    dd = mic_fast(pj.z - pi.z, 0.5f * Lz, Lz); r2 = fmaf(dd, dd, r2);
-    if (r2 <= rl2) {
-      if (found < cap) nbr[(size_t)found * N + i] = j + 1;
-      ++found;
+  if (active) {
+    const float Lx = geom[0], Ly = geom[1], Lz = geom[2];
+    const float4 pi = packed[i];
+    for (int j = 0; j < N; ++j) {
+      if (j == i) continue;
+      const float4 pj = packed[j];
+      // dimension order of the reference's loop: r2 = muladd(dd, dd, r2) for d = 1..D
+      float r2 = 0.0f;
+      float dd = mic_fast(pj.x - pi.x, 0.5f * Lx, Lx); r2 = fmaf(dd, dd, r2);
+      dd = mic_fast(pj.y - pi.y, 0.5f * Ly, Ly); r2 = fmaf(dd, dd, r2);
+      dd = mic_fast(pj.z - pi.z, 0.5f * Lz, Lz); r2 = fmaf(dd, dd, r2);
+      if (r2 <= rl2) {
+        if (found < cap) nbr[(size_t)found * N + i] = j + 1;
+        ++found;
+      }
     }
+    counts[i] = found;
+    if (candidates) candidates[i] = N - 1;
   }
-  counts[i] = found;
-  if (candidates) candidates[i] = N - 1;
+  row_partials(found, active ? N - 1 : 0, found, row_max, stat_partial);
 }
 
 // ------------------------------------------------------------------ commit
-// Largest row vs cap, build counters (_device_capacity_partial_kernel! + _device_commit_kernel!,
-// DeviceNeighborCUDA.jl:291-388), one launch with a last-block commit.
-__global__ __launch_bounds__(TPB) void k_commit(int N, const int32_t *counts, const int64_t *candidates,
-                                                 int32_t *partial, int64_t *stat_partial, const int64_t *state) {
+// Capacity commit (_device_commit_kernel!, DeviceNeighborCUDA.jl:291-388) and, when every row fitted,
+// the reference positions of the build. Every block reads the largest row; block 0 also adds the
+// statistics and writes the state words (the others need only the request and an error word that no
+// successful commit changes).
+__global__ __launch_bounds__(TPB) void k_commit_refs(int N, int nblocks, int cap, const int32_t *__restrict__ row_max,
+                                                     const int64_t *__restrict__ stat_partial,
+                                                     const float4 *__restrict__ packed, float *rref, int64_t *state) {
   if (!rebuild_requested(state)) return;
+  const int largest = *row_max;
   const int i = blockIdx.x * TPB + threadIdx.x;
-  const int v = i < N ? counts[i] : 0;
-  const int64_t cand = (candidates && i < N) ? candidates[i] : 0;
-  __shared__ int smax[TPB / WAVE];
+  if (largest <= cap && i < N) {
+    const float4 p = packed[i];
+    rref[i] = p.x;
+    rref[(size_t)N + i] = p.y;
+    rref[(size_t)2 * N + i] = p.z;
+  }
+  if (blockIdx.x != 0) return;
   __shared__ long long ssum[2][TPB / WAVE];
-  int m = wave_max(v);
-  long long sc = cand, sa = v;
-  for (int off = 32; off >= 1; off >>= 1) {
-    sc += __shfl_xor(sc, off, WAVE);
-    sa += __shfl_xor(sa, off, WAVE);
-  }
-  const int w = threadIdx.x / WAVE;
-  if ((threadIdx.x & (WAVE - 1)) == 0) { smax[w] = m; ssum[0][w] = sc; ssum[1][w] = sa; }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int b = smax[0]; long long c0 = ssum[0][0], a0 = ssum[1][0];
-    for (int k = 1; k < TPB / WAVE; ++k) { b = max(b, smax[k]); c0 += ssum[0][k]; a0 += ssum[1][k]; }
-    partial[blockIdx.x] = b;
-    stat_partial[2 * blockIdx.x] = c0;
-    stat_partial[2 * blockIdx.x + 1] = a0;
-  }
-}
-
-// Capacity commit from the blocks' partials (one wave64; integer sums, so any order is exact).
-__global__ __launch_bounds__(WAVE) void k_commit_final(int nblocks, int cap, const int32_t *__restrict__ partial,
-                                                       const int64_t *__restrict__ stat_partial, int64_t *state) {
-  if (!rebuild_requested(state)) return;
-  int largest = 0;
   long long ctot = 0, atot = 0;
-  for (int b = threadIdx.x; b < nblocks; b += WAVE) {
-    largest = max(largest, partial[b]);
+  for (int b = threadIdx.x; b < nblocks; b += TPB) {
     ctot += stat_partial[2 * b];
     atot += stat_partial[2 * b + 1];
   }
-  largest = wave_max(largest);
   for (int off = 32; off >= 1; off >>= 1) {
     ctot += __shfl_xor(ctot, off, WAVE);
     atot += __shfl_xor(atot, off, WAVE);
   }
+  const int w = threadIdx.x / WAVE;
+  if ((threadIdx.x & (WAVE - 1)) == 0) { ssum[0][w] = ctot; ssum[1][w] = atot; }
+  __syncthreads();
+  for (int k = 1; k < TPB / WAVE; ++k) { ctot += ssum[0][k]; atot += ssum[1][k]; }
   if (threadIdx.x != 0) return;
   state[PDX_DN_REQUIRED] = largest;
   const bool diag = state[PDX_DN_DIAGNOSTICS] != 0;
@@ -787,6 +957,7 @@ int enqueue_rebuild(pdx_nl_t nl, hipStream_t st) {
   const int nb = blocks_for(N, TPB);
   int64_t *s = nl->state.p;
   const float *geom = nl->geom.p;
+  int row_blocks = nb;  // workgroups of the row kernel, one commit partial each
   if (!nl->allpairs) {
     const int sblocks = blocks_for(nl->ncell, SCAN_BLOCK);
     hipLaunchKernelGGL(k_bin, dim3(nb), dim3(TPB), 0, st, N, nl->packed.p, geom, nl->nx, nl->ny, nl->nz,
@@ -805,7 +976,13 @@ int enqueue_rebuild(pdx_nl_t nl, hipStream_t st) {
                        nl->cell_offsets.p, nl->particle_ids_sorted.p, s);
     hipLaunchKernelGGL(k_sort_cells, dim3(std::min(nl->ncell, 8192)), dim3(WAVE), 0, st, nl->ncell, nl->cell_offsets.p,
                        nl->particle_ids_sorted.p, nl->packed.p, nl->sorted.p, s);
-    // lanes per particle: the list's row lanes; with PDX_ROW_STAGE=1 the rows are staged in LDS and
+    // The mask build, a workgroup per cell, where there are four cells a CU and cells of 14 particles
+    // and more on average. Whole rebuilds in microseconds, masks against k_rows at its default lanes
+    // (random particles in cell order): 4 096 cells of 2, 8, 14, 60 particles 80 / 90 / 103 / 628
+    // against 53 / 73 / 109 / 726; 21 952 cells of 4, 8, 14, 30: 140 / 176 / 282 / 665 against
+    // 102 / 152 / 330 / 988; 1 000 cells of 60: 230 against 208. k_rows also takes a caller's lane
+    // count and the opt-in forms below.
+    // Lanes per particle of k_rows: the list's row lanes; with PDX_ROW_STAGE=1 the rows are staged in LDS and
     // the lanes raised until the workgroup's rows fit the 64 KiB stage. Staging cuts the build's HBM
     // writes at 486 400 ions from 3.97 GB to 0.93 GB but not its time (1.13 ms at 32 lanes against
     // 1.12 ms written straight at 8), so the default writes straight from the search.
@@ -820,12 +997,19 @@ int enqueue_rebuild(pdx_nl_t nl, hipStream_t st) {
     bool cells = false;
     if (const char *v = std::getenv("PDX_ROW_CELLS")) cells = std::atoi(v) != 0;
     if (stage) cells = false;
-    if (cells) {
+    const bool masks = !stage && !cells && !nl->row_lanes_given && nl->ncell >= 1024 && N >= 14 * (int64_t)nl->ncell;
+    if (masks) {
+      row_blocks = std::min(nl->ncell, 4096);
+      hipLaunchKernelGGL(k_rows_masks, dim3(row_blocks), dim3(TPB), 0, st, N, nl->cap, nl->ncell, nl->nx, nl->ny,
+                         nl->nz, nl->sorted.p, nl->cell_offsets.p, geom, nl->rl2, nl->neighbors_flat.p, nl->counts.p,
+                         nl->diagnostics ? nl->candidates.p : nullptr, nl->row_max.p, nl->stat_partial.p, s);
+    } else if (cells) {
+      row_blocks = std::min(nl->ncell, 8192);
 #define PDX_ROWC(GG)                                                                                        \
-  hipLaunchKernelGGL((k_rows_cells<GG>), dim3(std::min(nl->ncell, 8192)), dim3(TPB), 0, st, N, nl->cap, nl->ncell, \
+  hipLaunchKernelGGL((k_rows_cells<GG>), dim3(row_blocks), dim3(TPB), 0, st, N, nl->cap, nl->ncell, \
                      nl->nx, nl->ny, nl->nz, \
                      nl->sorted.p, nl->cell_offsets.p, geom, nl->rl2, nl->neighbors_flat.p, nl->counts.p,     \
-                     nl->diagnostics ? nl->candidates.p : nullptr, s);
+                     nl->diagnostics ? nl->candidates.p : nullptr, nl->row_max.p, nl->stat_partial.p, s);
       switch (G) {
         case 1: PDX_ROWC(1) break;
         case 2: PDX_ROWC(2) break;
@@ -843,16 +1027,19 @@ int enqueue_rebuild(pdx_nl_t nl, hipStream_t st) {
       else stage = false;
     }
     const int rb = (int)(((int64_t)N * G + TPB - 1) / TPB);
+    row_blocks = rb;
     const size_t lds = stage ? (size_t)(TPB / G) * nl->cap * sizeof(int32_t) : 0;
 #define PDX_ROWS(GG)                                                                                       \
   if (stage)                                                                                               \
     hipLaunchKernelGGL((k_rows<GG, true>), dim3(rb), dim3(TPB), lds, st, N, nl->cap, nl->nx, nl->ny, nl->nz, \
                        nl->sorted.p, nl->cell_offsets.p, nl->cell_of_particle.p, geom, nl->rl2,            \
-                       nl->neighbors_flat.p, nl->counts.p, nl->diagnostics ? nl->candidates.p : nullptr, s); \
+                       nl->neighbors_flat.p, nl->counts.p, nl->diagnostics ? nl->candidates.p : nullptr,   \
+                       nl->row_max.p, nl->stat_partial.p, s);                                          \
   else                                                                                                     \
     hipLaunchKernelGGL((k_rows<GG, false>), dim3(rb), dim3(TPB), 0, st, N, nl->cap, nl->nx, nl->ny, nl->nz, \
                        nl->sorted.p, nl->cell_offsets.p, nl->cell_of_particle.p, geom, nl->rl2,            \
-                       nl->neighbors_flat.p, nl->counts.p, nl->diagnostics ? nl->candidates.p : nullptr, s);
+                       nl->neighbors_flat.p, nl->counts.p, nl->diagnostics ? nl->candidates.p : nullptr,   \
+                       nl->row_max.p, nl->stat_partial.p, s);
     switch (G) {
       case 1: PDX_ROWS(1) break;
       case 2: PDX_ROWS(2) break;
@@ -866,12 +1053,10 @@ int enqueue_rebuild(pdx_nl_t nl, hipStream_t st) {
   } else {
     hipLaunchKernelGGL(k_rows_allpairs, dim3(nb), dim3(TPB), 0, st, N, nl->cap, nl->packed.p, geom,
                        nl->rl2, nl->neighbors_flat.p, nl->counts.p,
-                       nl->diagnostics ? nl->candidates.p : nullptr, s);
+                       nl->diagnostics ? nl->candidates.p : nullptr, nl->row_max.p, nl->stat_partial.p, s);
   }
-  hipLaunchKernelGGL(k_commit, dim3(nb), dim3(TPB), 0, st, N, nl->counts.p,
-                     nl->diagnostics ? nl->candidates.p : nullptr, nl->cap_partial.p, nl->stat_partial.p, s);
-  hipLaunchKernelGGL(k_commit_final, dim3(1), dim3(64), 0, st, nb, nl->cap, nl->cap_partial.p, nl->stat_partial.p, s);
-  hipLaunchKernelGGL(k_copy_refs, dim3(nb), dim3(TPB), 0, st, N, nl->packed.p, nl->rref.p, s);
+  hipLaunchKernelGGL(k_commit_refs, dim3(nb), dim3(TPB), 0, st, N, row_blocks, nl->cap, nl->row_max.p,
+                     nl->stat_partial.p, nl->packed.p, nl->rref.p, s);
   PDX_LAUNCH_CHECK();
   return PDX_OK;
 }
@@ -886,12 +1071,12 @@ int enqueue_check(pdx_nl_t nl, const float *x, const float *y, const float *z, c
   float *xw = const_cast<float *>(x), *yw = const_cast<float *>(y), *zw = const_cast<float *>(z);
   if (kd)
     hipLaunchKernelGGL(k_decide<true>, dim3(nb), dim3(TPB), 0, st, N, xw, yw, zw, q, nl->rref.p, nl->packed.p,
-                       nl->cell_counts.p, nl->ncell, (int)nl->allpairs, nl->geom.p, nl->state.p, nl->disp_partial.p,
+                       nl->cell_counts.p, nl->row_max.p, nl->ncell, (int)nl->allpairs, nl->geom.p, nl->state.p, nl->disp_partial.p,
                        (const int32_t *)nl->cell_offsets.p, (const int32_t *)nl->particle_ids_sorted.p,
                        nl->snap_offsets.p, nl->snap_ids.p, nl->snap_state.p, *kd);
   else
     hipLaunchKernelGGL(k_decide<false>, dim3(nb), dim3(TPB), 0, st, N, xw, yw, zw, q, nl->rref.p, nl->packed.p,
-                       nl->cell_counts.p, nl->ncell, (int)nl->allpairs, nl->geom.p, nl->state.p, nl->disp_partial.p,
+                       nl->cell_counts.p, nl->row_max.p, nl->ncell, (int)nl->allpairs, nl->geom.p, nl->state.p, nl->disp_partial.p,
                        (const int32_t *)nl->cell_offsets.p, (const int32_t *)nl->particle_ids_sorted.p,
                        nl->snap_offsets.p, nl->snap_ids.p, nl->snap_state.p, KickDrift{});
   PDX_LAUNCH_CHECK();
@@ -982,20 +1167,24 @@ extern "C" int pdx_nl_create(int32_t n, const double box[3], double cutoff, doub
     while (G < 32 && cand > 256.0 * G) G <<= 1;
     if (const char *v = std::getenv("PDX_ROW_LANES")) {
       const int e = std::atoi(v);
-      if (e == 1 || e == 2 || e == 4 || e == 8 || e == 16 || e == 32) G = e;
+      if (e == 1 || e == 2 || e == 4 || e == 8 || e == 16 || e == 32) {
+        G = e;
+        nl->row_lanes_given = true;
+      }
     }
     nl->row_lanes = G;
   }
   const int nb = blocks_for(n, TPB);
   nl->ndisp = nb;
+  const int cb = std::max(blocks_for((int64_t)n * 32, TPB), 8192);  // the row kernels' largest grids
   const int sblocks = blocks_for(nl->ncell, SCAN_BLOCK);
   if ((rc = nl->state.alloc(PDX_DN_NSTATE)) || (rc = nl->geom.alloc(3)) ||
       (rc = nl->neighbors_flat.alloc((size_t)n * cap)) || (rc = nl->counts.alloc(n)) ||
       (rc = nl->cell_offsets.alloc(nl->ncell + 1)) || (rc = nl->cell_counts.alloc(nl->ncell)) ||
       (rc = nl->particle_ids_sorted.alloc(n)) || (rc = nl->cell_of_particle.alloc(n)) ||
       (rc = nl->cell_rank.alloc(n)) || (rc = nl->rref.alloc((size_t)3 * n)) || (rc = nl->packed.alloc(n)) ||
-      (rc = nl->sorted.alloc(n)) || (rc = nl->sortedq.alloc(n)) || (rc = nl->disp_partial.alloc(nb)) || (rc = nl->cap_partial.alloc(nb)) ||
-      (rc = nl->stat_partial.alloc((size_t)2 * nb)) || (rc = nl->scan_block.alloc(sblocks)) ||
+      (rc = nl->sorted.alloc(n)) || (rc = nl->sortedq.alloc(n)) || (rc = nl->disp_partial.alloc(nb)) || (rc = nl->row_max.alloc(1)) ||
+      (rc = nl->stat_partial.alloc((size_t)2 * cb)) || (rc = nl->scan_block.alloc(sblocks)) ||
       (rc = nl->candidates.alloc(nl->diagnostics ? n : 1)) ||
       (rc = nl->snap_offsets.alloc((size_t)nl->ncell + 1)) || (rc = nl->snap_ids.alloc(n)) ||
       (rc = nl->snap_state.alloc(4))) {
@@ -1251,5 +1440,6 @@ extern "C" int pdx_nl_set_row_lanes(pdx_nl_t nl, int32_t lanes) {
   if (lanes != 1 && lanes != 2 && lanes != 4 && lanes != 8 && lanes != 16 && lanes != 32)
     return fail(PDX_ERR_ARGUMENT, "row-build lanes must be 1, 2, 4, 8, 16 or 32");
   nl->row_lanes = lanes;
+  nl->row_lanes_given = true;
   return PDX_OK;
 }

@@ -220,3 +220,50 @@ def test_rows_staged_equal_direct_and_lanes(cuda, case, monkeypatch):
     for lanes in (None, 1, 4, 8, 32):
         c1, r1, _ = rows(False, lanes, cells=True)
         assert torch.equal(c0, c1) and torch.equal(r0, r1), ("cells", lanes)
+
+
+@pytest.mark.parametrize("grid", [(3, 18, 20), (4, 16, 17), (5, 14, 15), (10, 11, 12)])
+@pytest.mark.parametrize("clump", [0, 2200])
+def test_rows_of_dense_cells_equal_row_search(cuda, grid, clump):
+    """The cell-wise build that many well-filled cells take by default (at least 1 024 cells of 14
+    particles and more) writes the rows, slot for slot, the candidate counts and the statistics of the
+    row search (an explicit lane count): grids with and without cells off the seam, particles on the
+    box faces, a clump with more particles in a cell than a wavefront has lanes and more candidates
+    than one pass holds, and rows longer than the capacity."""
+    import torch
+    w, cutoff, skin = 3.001, 2.5, 0.5
+    box = tuple(w * g for g in grid)
+    rng = np.random.default_rng(sum(grid) + clump)
+    n0 = 14 * int(np.prod(grid)) + 37
+    p = (rng.random((n0, 3)) - 0.5) * np.array(box)
+    for d in range(3):  # on the faces, and next to where the face's image reaches
+        p[20 * d:20 * d + 10, d] = np.float32(0.5 * box[d])
+        p[20 * d + 10:20 * d + 20, d] = -0.5 * box[d] + w * (1 - 1e-4 * rng.random(10))
+    if clump:
+        at = np.array([0.5 * box[0] - 0.1, 0.3, -0.7])
+        q = at + 2.2 * w * (rng.random((clump, 3)) - 0.5)
+        q[:150] = at - 0.08 * rng.random((150, 3))
+        q -= np.array(box) * np.round(q / np.array(box))
+        p = np.concatenate([p, q])
+    h = np.float32(0.5) * np.array(box, dtype=np.float32)
+    p = np.clip(p.astype(np.float32), -h, h)
+    N = len(p)
+    X, Y, Z = (dev(np.ascontiguousarray(p[:, d])) for d in range(3))
+    for cap in (N if N < 2000 else 1500, 40):
+        out = []
+        for lanes in (None, 4):
+            ws = pdx.DeviceNeighborWorkspace(N, box, cutoff, skin, cap)
+            if lanes:
+                ws.set_row_lanes(lanes)
+            assert (ws.nx, ws.ny, ws.nz) == grid and ws.ncell >= 1024 and N >= 14 * ws.ncell
+            print(f"[rows] {grid} N={N} cap={cap} lanes={lanes}", flush=True)
+            ws.update(X, Y, Z, None)
+            st = ws.state()
+            cnt = ws.counts().clone()
+            flat = ws.neighbors_flat().clone()
+            keep = torch.arange(cap, device="cuda")[:, None] < cnt[None, :]
+            out.append((cnt, torch.where(keep, flat, torch.zeros_like(flat)), st))
+        (c0, r0, s0), (c1, r1, s1) = out
+        assert torch.equal(c0, c1) and torch.equal(r0, r1)
+        assert s0 == s1
+        assert (int(c0.max()) > cap) == (s0[2] != 0) and s0[8] == int(c0.max())
