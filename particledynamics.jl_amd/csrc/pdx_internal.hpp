@@ -295,6 +295,7 @@ struct pdx_nl_s {
   pdx::DevBuf<float4> sortedq;  // N, cell order, current (x, y, z, q): the cell traversal's copy
   pdx::DevBuf<float> disp_partial;  // ndisp per-block maxima of the last check
   int32_t ndisp = 0;
+  pdx::DevBuf<int64_t> decision;      // the check's decision on its way to the state words
   pdx::DevBuf<int32_t> row_max;       // largest row of the build under way
   pdx::DevBuf<int64_t> stat_partial;  // 2 per row block: candidates, accepted
   pdx::DevBuf<int32_t> scan_block;    // per-1024-cell block totals

@@ -5,11 +5,11 @@
 // hipGraph — the "predicated reference path" of src/neighbors/DeviceNeighborCUDA.jl:413-420):
 //   k_decide       coverage check: per-block max |dr|^2, packing of (x, y, z, q), zeroing of
 //                  the cell histogram
-//   k_decide_final max over the blocks vs skin^2/4, age, adaptive interval (one block)
+//   k_decide_final max over the blocks vs skin^2/4, age, adaptive interval (one block); lists of up to
+//                  DECIDE_BLOCKS check blocks and SCAN_FUSED_MAX cells decide in k_bin instead
 //   k_bin          cell id + histogram; the atomic's return value is the particle's slot
-//   k_scan_single  (or k_scan_local / k_scan_blocks / k_scan_finish above 16384 cells)
-//                  exclusive scan -> 1-based cell_offsets
-//   k_scatter      particle_ids_sorted (1-based)
+//   k_scan_scatter exclusive scan -> 1-based cell_offsets, particle_ids_sorted (1-based)
+//                  (k_scan_local / k_scan_blocks / k_scan_finish / k_scatter above SCAN_FUSED_MAX cells)
 //   k_sort_cells   ascending id inside each cell (rows and traversal become reproducible),
 //                  and the cell-ordered packed positions read by the row kernel
 //   k_rows_masks   (or k_rows / k_rows_cells / k_rows_allpairs) 27-cell stencil, r^2 <= rlist^2,
@@ -26,6 +26,7 @@ using namespace pdx;
 namespace {
 
 constexpr int TPB = 256;
+constexpr int DECIDE_BLOCKS = 1024;  // check blocks of a list whose k_bin decides
 constexpr int SCAN_BLOCK = 1024;  // cells per block of the local scan (256 threads x 4)
 
 __device__ __forceinline__ bool rebuild_requested(const int64_t *s) {
@@ -46,7 +47,7 @@ struct KickDrift {
 
 // Coverage check (_device_displacement_kernel! + _device_decide_kernel!,
 // DeviceNeighborCUDA.jl:169-236): per-block maximum squared displacement (plus the float4
-// packing and the histogram clearing), then one block decides (k_decide_final). With KD the
+// packing and the histogram clearing), then k_decide_final or k_bin decides. With KD the
 // step's kick-drift moves x, y, z (in place) first.
 template <bool KD>
 __global__ __launch_bounds__(TPB) void k_decide(int N, float *__restrict__ x,
@@ -63,12 +64,12 @@ __global__ __launch_bounds__(TPB) void k_decide(int N, float *__restrict__ x,
   if (err != 0) return;  // latched: every block leaves (uniform)
   const int i = blockIdx.x * TPB + threadIdx.x;
   // cell snapshot: the cells of a build completed since the last snapshot, copied before this
-  // step's rebuild can overwrite them (k_decide_final records the build); a spread on another
+  // step's rebuild can overwrite them (the decision records the build); a spread on another
   // stream may then read them beside the rebuild
   if (!allpairs && state[PDX_DN_BUILDS] > 0 && state[PDX_DN_BUILDS] != snap[0]) {
     for (int c = i; c <= ncell; c += gridDim.x * TPB) snap_offsets[c] = offsets[c];
     if (i < N) snap_ids[i] = ids[i];
-    if (i == 0) snap[2] = 0;  // valid once this launch completes (snap[0] is written by k_decide_final)
+    if (i == 0) snap[2] = 0;  // valid once this launch completes (snap[0] is written with the decision)
   }
   const float L[3] = {geom[0], geom[1], geom[2]};
   const bool valid = state[PDX_DN_VALID] != 0;
@@ -123,63 +124,102 @@ __global__ __launch_bounds__(TPB) void k_decide(int N, float *__restrict__ x,
   }
 }
 
-// The decision from the blocks' maxima (one block).
-__global__ __launch_bounds__(TPB) void k_decide_final(int nblocks, const float *__restrict__ partial, int64_t *state,
-                                                       float threshold, int force, int64_t *snap, int allpairs) {
-  if (state[PDX_DN_ERROR] != 0) return;
+// Largest of the check blocks' maxima (every thread of the block).
+__device__ __forceinline__ float largest_displacement(int nblocks, const float *__restrict__ partial) {
   __shared__ float smax[TPB / WAVE];
   float v = 0.0f;
   for (int b = threadIdx.x; b < nblocks; b += TPB) v = fmaxf(v, partial[b]);
   v = wave_max(v);
   if ((threadIdx.x & (WAVE - 1)) == 0) smax[threadIdx.x / WAVE] = v;
   __syncthreads();
-  if (threadIdx.x != 0) return;
-  if (!allpairs && state[PDX_DN_BUILDS] > 0 && state[PDX_DN_BUILDS] != snap[0])  // k_decide copied it
-    snap[0] = state[PDX_DN_BUILDS];
   float largest = smax[0];
   for (int w = 1; w < TPB / WAVE; ++w) largest = fmaxf(largest, smax[w]);
-  const bool valid = state[PDX_DN_VALID] != 0;
-  state[PDX_DN_CHECKS] += 1;
-  state[PDX_DN_REQUEST] = 0;
-  const bool diag = state[PDX_DN_DIAGNOSTICS] != 0;
-  if (diag) state[PDX_DN_REASON] = 0;
+  return largest;
+}
+
+// What the decision makes of the state words (read only).
+struct Decision {
+  int64_t active;  // 0: an error is latched, nothing changes
+  int64_t request, valid, error, reason, interval;
+};
+__device__ __forceinline__ Decision decide(float largest, const int64_t *state, float threshold, int force) {
+  Decision d{state[PDX_DN_ERROR] == 0, 0, state[PDX_DN_VALID], state[PDX_DN_ERROR], 0, state[PDX_DN_INTERVAL]};
   if (!isfinite(largest)) {
-    state[PDX_DN_ERROR] = PDX_DN_COORDINATE_ERROR;
-    state[PDX_DN_VALID] = 0;
-    return;
+    d.error = PDX_DN_COORDINATE_ERROR;
+    d.valid = 0;
+    return d;
   }
-  if (force || !valid) {
-    state[PDX_DN_REQUEST] = 1;
-    state[PDX_DN_VALID] = 0;
-    if (diag) state[PDX_DN_REASON] = PDX_DN_REASON_INVALID;
-    return;
+  if (force || d.valid == 0) {
+    d.request = 1;
+    d.valid = 0;
+    d.reason = PDX_DN_REASON_INVALID;
+    return d;
   }
   const int64_t age = state[PDX_DN_STEP] - state[PDX_DN_LAST_BUILD];
   const bool disp = largest > threshold;
-  const bool old = age >= state[PDX_DN_INTERVAL];
+  const bool old = age >= d.interval;
   if (disp || old) {
-    state[PDX_DN_REQUEST] = 1;
-    state[PDX_DN_VALID] = 0;
-    if (diag) state[PDX_DN_REASON] = (disp ? PDX_DN_REASON_DISPLACEMENT : 0) | (old ? PDX_DN_REASON_AGE : 0);
+    d.request = 1;
+    d.valid = 0;
+    d.reason = (disp ? PDX_DN_REASON_DISPLACEMENT : 0) | (old ? PDX_DN_REASON_AGE : 0);
     // adaptive interval: x0.9 on displacement, x1.1 when the list aged out early, in [5, 100]
     if (disp) {
-      float t = rintf(0.9f * (float)state[PDX_DN_INTERVAL]);
-      state[PDX_DN_INTERVAL] = t < 5.0f ? 5 : (int64_t)t;
+      float t = rintf(0.9f * (float)d.interval);
+      d.interval = t < 5.0f ? 5 : (int64_t)t;
     } else if (largest < 0.1f * threshold) {
-      float t = rintf(1.1f * (float)state[PDX_DN_INTERVAL]);
-      state[PDX_DN_INTERVAL] = t > 100.0f ? 100 : (int64_t)t;
+      float t = rintf(1.1f * (float)d.interval);
+      d.interval = t > 100.0f ? 100 : (int64_t)t;
     }
   }
+  return d;
+}
+__device__ __forceinline__ void write_decision(const Decision &d, int64_t *state) {
+  state[PDX_DN_CHECKS] += 1;
+  state[PDX_DN_REQUEST] = d.request;
+  if (state[PDX_DN_DIAGNOSTICS] != 0) state[PDX_DN_REASON] = d.reason;
+  state[PDX_DN_ERROR] = d.error;
+  state[PDX_DN_VALID] = d.valid;
+  state[PDX_DN_INTERVAL] = d.interval;
+}
+// The check's snapshot (k_decide copied it) is of this build.
+__device__ __forceinline__ void record_snapshot(const int64_t *state, int64_t *snap) {
+  if (state[PDX_DN_BUILDS] > 0 && state[PDX_DN_BUILDS] != snap[0]) snap[0] = state[PDX_DN_BUILDS];
+}
+
+// The decision from the blocks' maxima (one block).
+__global__ __launch_bounds__(TPB) void k_decide_final(int nblocks, const float *__restrict__ partial, int64_t *state,
+                                                       float threshold, int force, int64_t *snap, int allpairs) {
+  if (state[PDX_DN_ERROR] != 0) return;
+  const float largest = largest_displacement(nblocks, partial);
+  if (threadIdx.x != 0) return;
+  if (!allpairs) record_snapshot(state, snap);
+  write_decision(decide(largest, state, threshold, force), state);
 }
 
 // ------------------------------------------------------------------ binning
 // Cell id from the current box, fractional binning floor(x n/L) (_kernel_cell_ids3g!,
 // DeviceNeighborCUDA.jl:464-481) + histogram (_kernel_cell_histogram!, DenseNeighborCUDA.jl:50).
+// DECIDE: every block takes the decision itself from the check's partials and the state words, which
+// no block of this launch writes; block 0 hands it to k_scan_scatter, which writes the words. A launch
+// that finds nothing to do is 4-5 us of a step: with this and k_scan_scatter's fusion a step of 256 000 LJ
+// atoms went from 98 to 96 us, an eager evaluation of 4 000 atoms from 40 to 32 us.
+template <bool DECIDE>
 __global__ __launch_bounds__(TPB) void k_bin(int N, const float4 *__restrict__ packed,
                                               const float *geom, int nx, int ny, int nz,
                                               int32_t *cell_of_particle, int32_t *cell_counts,
-                                              int32_t *cell_rank, const int64_t *state) {
-  if (!rebuild_requested(state)) return;
+                                              int32_t *cell_rank, const int64_t *state, int nblocks,
+                                              const float *__restrict__ partial, float threshold, int force,
+                                              int64_t *snap, Decision *decision) {
+  if (DECIDE) {
+    const Decision d = decide(largest_displacement(nblocks, partial), state, threshold, force);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      *decision = d;
+      if (d.active) record_snapshot(state, snap);
+    }
+    if (!d.active || !d.request) return;
+  } else if (!rebuild_requested(state)) {
+    return;
+  }
   const int i = blockIdx.x * TPB + threadIdx.x;
   if (i >= N) return;
   const float4 p = packed[i];
@@ -195,18 +235,38 @@ __global__ __launch_bounds__(TPB) void k_bin(int N, const float4 *__restrict__ p
   cell_rank[i] = atomicAdd(&cell_counts[c], 1);
 }
 
-// Cell offsets in one launch for grids of up to 16384 cells: 1024 threads, a contiguous run of
-// at most 16 cells each, wave scans of the run totals; 1-based, last entry N+1
-// (_device_offsets_kernel!, DeviceNeighborCUDA.jl:280-289).
-constexpr int SCAN_SINGLE_MAX = 16384;
-__global__ __launch_bounds__(1024) void k_scan_single(int ncell, int N, const int32_t *__restrict__ counts,
-                                                       int32_t *offsets, const int64_t *state) {
-  if (!rebuild_requested(state)) return;
-  __shared__ int32_t wtot[16];
-  const int per = (ncell + 1023) / 1024;
-  const int c0 = min(threadIdx.x * per, ncell), c1 = min(c0 + per, ncell);
+// Cell offsets (1-based, last entry N+1: _device_offsets_kernel!, DeviceNeighborCUDA.jl:280-289) and
+// the particles' scatter in one launch for grids of up to SCAN_FUSED_MAX cells: every workgroup scans
+// all counts in its LDS (1024 threads, a contiguous run of at most 16 cells each, wave scans of the
+// run totals; the counts come from the caches) and places its share of the particles; workgroup 0
+// stores the offsets and, with DECIDE, writes k_bin's decision into the state words, which the other
+// workgroups do not read.
+constexpr int SCAN_FUSED_MAX = 16000;  // 62.5 KiB of LDS
+constexpr int SCAN_THREADS = 1024;
+constexpr int SCAN_GRID = 64;  // 16 and 256 are 1% slower (256 000 LJ atoms), 1 is 10%
+template <bool DECIDE>
+__global__ __launch_bounds__(SCAN_THREADS) void k_scan_scatter(int ncell, int N, const int32_t *__restrict__ counts,
+                                                               int32_t *offsets,
+                                                               const int32_t *__restrict__ cell_of_particle,
+                                                               const int32_t *__restrict__ cell_rank,
+                                                               int32_t *ids_sorted, int64_t *state,
+                                                               const Decision *__restrict__ decision) {
+  if (DECIDE) {
+    const Decision d = *decision;
+    if (!d.active) return;
+    if (blockIdx.x == 0 && threadIdx.x == 0) write_decision(d, state);
+    if (!d.request) return;
+  } else if (!rebuild_requested(state)) {
+    return;
+  }
+  extern __shared__ int32_t first[];  // ncell
+  __shared__ int32_t wtot[SCAN_THREADS / WAVE];
+  for (int c = threadIdx.x; c < ncell; c += SCAN_THREADS) first[c] = counts[c];
+  __syncthreads();
+  const int per = (ncell + SCAN_THREADS - 1) / SCAN_THREADS;
+  const int c0 = min((int)threadIdx.x * per, ncell), c1 = min(c0 + per, ncell);
   int32_t run = 0;
-  for (int c = c0; c < c1; ++c) run += counts[c];
+  for (int c = c0; c < c1; ++c) run += first[c];
   const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
   int32_t v = run;
 #pragma unroll
@@ -219,10 +279,17 @@ __global__ __launch_bounds__(1024) void k_scan_single(int ncell, int N, const in
   int32_t base = v - run + 1;
   for (int k = 0; k < w; ++k) base += wtot[k];
   for (int c = c0; c < c1; ++c) {
-    offsets[c] = base;
-    base += counts[c];
+    const int32_t n = first[c];
+    first[c] = base;
+    base += n;
   }
-  if (threadIdx.x == 0) offsets[ncell] = N + 1;
+  __syncthreads();
+  if (blockIdx.x == 0) {
+    for (int c = threadIdx.x; c < ncell; c += SCAN_THREADS) offsets[c] = first[c];
+    if (threadIdx.x == 0) offsets[ncell] = N + 1;
+  }
+  for (int i = blockIdx.x * SCAN_THREADS + threadIdx.x; i < N; i += gridDim.x * SCAN_THREADS)
+    ids_sorted[first[cell_of_particle[i]] - 1 + cell_rank[i]] = i + 1;
 }
 
 // Exclusive scan of cell_counts, SCAN_BLOCK cells per block (block-local part).
@@ -952,28 +1019,46 @@ int grid_for_box(const double box[3], double rl, int32_t out[3]) {
   return PDX_OK;
 }
 
-int enqueue_rebuild(pdx_nl_t nl, hipStream_t st) {
+// The decision from the check's partial maxima (and the snapshot's record), then the predicated
+// rebuild.
+int enqueue_decide_build(pdx_nl_t nl, hipStream_t st) {
   const int N = nl->N;
   const int nb = blocks_for(N, TPB);
   int64_t *s = nl->state.p;
   const float *geom = nl->geom.p;
+  const float skin = (float)nl->skin;
+  const float threshold = (0.25f * skin) * skin;
   int row_blocks = nb;  // workgroups of the row kernel, one commit partial each
+  // k_bin decides where its workgroups reread at most 1 024 partials each (4 KB, from the caches) and
+  // k_scan_scatter follows to write the decision down; else a launch of its own does. Forty steps of
+  // 256 000 LJ atoms (1 000 blocks): 3.67 ms in k_bin, 3.74 apart; a pass of 7 600 ions 78 and 82 us;
+  // forty steps of 486 400 ions (1 900 blocks, beside the mesh): 23.2 ms in k_bin, 22.9 apart
+  const bool scan_fused = !nl->allpairs && nl->ncell <= SCAN_FUSED_MAX;
+  const bool decide_fused = scan_fused && nb <= DECIDE_BLOCKS;
+  Decision *dec = (Decision *)nl->decision.p;
+  if (!decide_fused)
+    hipLaunchKernelGGL(k_decide_final, dim3(1), dim3(TPB), 0, st, nb, nl->disp_partial.p, s, threshold,
+                       nl->check_force, nl->snap_state.p, (int)nl->allpairs);
   if (!nl->allpairs) {
     const int sblocks = blocks_for(nl->ncell, SCAN_BLOCK);
-    hipLaunchKernelGGL(k_bin, dim3(nb), dim3(TPB), 0, st, N, nl->packed.p, geom, nl->nx, nl->ny, nl->nz,
-                       nl->cell_of_particle.p, nl->cell_counts.p, nl->cell_rank.p, s);
-    if (nl->ncell <= SCAN_SINGLE_MAX) {
-      hipLaunchKernelGGL(k_scan_single, dim3(1), dim3(1024), 0, st, nl->ncell, N, nl->cell_counts.p,
-                         nl->cell_offsets.p, s);
+    auto bin = decide_fused ? k_bin<true> : k_bin<false>;
+    hipLaunchKernelGGL(bin, dim3(nb), dim3(TPB), 0, st, N, nl->packed.p, geom, nl->nx, nl->ny, nl->nz,
+                       nl->cell_of_particle.p, nl->cell_counts.p, nl->cell_rank.p, s, nb, nl->disp_partial.p,
+                       threshold, nl->check_force, nl->snap_state.p, dec);
+    if (scan_fused) {
+      auto scan = decide_fused ? k_scan_scatter<true> : k_scan_scatter<false>;
+      hipLaunchKernelGGL(scan, dim3(std::min(blocks_for(N, SCAN_THREADS), SCAN_GRID)), dim3(SCAN_THREADS),
+                         sizeof(int32_t) * (size_t)nl->ncell, st, nl->ncell, N, nl->cell_counts.p, nl->cell_offsets.p,
+                         nl->cell_of_particle.p, nl->cell_rank.p, nl->particle_ids_sorted.p, s, dec);
     } else {
       hipLaunchKernelGGL(k_scan_local, dim3(sblocks), dim3(TPB), 0, st, nl->ncell, nl->cell_counts.p,
                          nl->cell_offsets.p, nl->scan_block.p, s);
       hipLaunchKernelGGL(k_scan_blocks, dim3(1), dim3(1024), 0, st, sblocks, nl->scan_block.p, s);
       hipLaunchKernelGGL(k_scan_finish, dim3(blocks_for(nl->ncell + 1, TPB)), dim3(TPB), 0, st, nl->ncell, N,
                          nl->cell_offsets.p, nl->scan_block.p, s);
+      hipLaunchKernelGGL(k_scatter, dim3(nb), dim3(TPB), 0, st, N, nl->cell_of_particle.p, nl->cell_rank.p,
+                         nl->cell_offsets.p, nl->particle_ids_sorted.p, s);
     }
-    hipLaunchKernelGGL(k_scatter, dim3(nb), dim3(TPB), 0, st, N, nl->cell_of_particle.p, nl->cell_rank.p,
-                       nl->cell_offsets.p, nl->particle_ids_sorted.p, s);
     hipLaunchKernelGGL(k_sort_cells, dim3(std::min(nl->ncell, 8192)), dim3(WAVE), 0, st, nl->ncell, nl->cell_offsets.p,
                        nl->particle_ids_sorted.p, nl->packed.p, nl->sorted.p, s);
     // The mask build, a workgroup per cell, where there are four cells a CU and cells of 14 particles
@@ -1086,18 +1171,6 @@ int enqueue_check(pdx_nl_t nl, const float *x, const float *y, const float *z, c
   return PDX_OK;
 }
 
-// The decision from the check's partial maxima (and the snapshot's record), then the
-// predicated rebuild.
-int enqueue_decide_build(pdx_nl_t nl, hipStream_t st) {
-  const float s = (float)nl->skin;
-  const float threshold = (0.25f * s) * s;
-  const int nb = blocks_for(nl->N, TPB);
-  hipLaunchKernelGGL(k_decide_final, dim3(1), dim3(TPB), 0, st, nb, nl->disp_partial.p, nl->state.p, threshold,
-                     nl->check_force, nl->snap_state.p, (int)nl->allpairs);
-  PDX_LAUNCH_CHECK();
-  return enqueue_rebuild(nl, st);
-}
-
 int enqueue_update(pdx_nl_t nl, const float *x, const float *y, const float *z, const float *q,
                    hipStream_t st, int force) {
   int rc = enqueue_check(nl, x, y, z, q, st, force);
@@ -1184,6 +1257,7 @@ extern "C" int pdx_nl_create(int32_t n, const double box[3], double cutoff, doub
       (rc = nl->particle_ids_sorted.alloc(n)) || (rc = nl->cell_of_particle.alloc(n)) ||
       (rc = nl->cell_rank.alloc(n)) || (rc = nl->rref.alloc((size_t)3 * n)) || (rc = nl->packed.alloc(n)) ||
       (rc = nl->sorted.alloc(n)) || (rc = nl->sortedq.alloc(n)) || (rc = nl->disp_partial.alloc(nb)) || (rc = nl->row_max.alloc(1)) ||
+      (rc = nl->decision.alloc(sizeof(Decision) / sizeof(int64_t))) ||
       (rc = nl->stat_partial.alloc((size_t)2 * cb)) || (rc = nl->scan_block.alloc(sblocks)) ||
       (rc = nl->candidates.alloc(nl->diagnostics ? n : 1)) ||
       (rc = nl->snap_offsets.alloc((size_t)nl->ncell + 1)) || (rc = nl->snap_ids.alloc(n)) ||

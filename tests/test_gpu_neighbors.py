@@ -267,3 +267,51 @@ def test_rows_of_dense_cells_equal_row_search(cuda, grid, clump):
         assert torch.equal(c0, c1) and torch.equal(r0, r1)
         assert s0 == s1
         assert (int(c0.max()) > cap) == (s0[2] != 0) and s0[8] == int(c0.max())
+
+
+@pytest.mark.parametrize("grid,N", [((3, 3, 3), 1), ((4, 5, 6), 1025), ((24, 24, 24), 262144), ((24, 24, 24), 262145),
+                                    ((20, 20, 40), 65537), ((20, 20, 41), 65537)])
+def test_cell_order_at_the_launch_rules(cuda, grid, N):
+    """Cells, offsets and sorted ids of a build, and the decision to build, on both sides of the sizes
+    where the binning takes the decision (262 144 particles) and the scan shares the scatter's launch
+    (16 000 cells)."""
+    import torch
+    w = 3.001
+    box = tuple(w * g for g in grid)
+    rng = np.random.default_rng(N + grid[2])
+    p = ((rng.random((N, 3)) - 0.5) * np.array(box)).astype(np.float32)
+    X, Y, Z = (dev(np.ascontiguousarray(p[:, d])) for d in range(3))
+    ws = pdx.DeviceNeighborWorkspace(N, box, 0.5, 2.5, min(max(N - 1, 1), 160))
+    print(f"[rows] {grid} N={N}", flush=True)
+
+    def check():
+        cell = ws.cell_of_particle().long()
+        edge = 1e-5 * np.array(grid)
+        f = [(torch.stack((X, Y, Z))[d].double() / box[d] + 0.5) * grid[d] for d in range(3)]
+        inside = torch.ones(N, dtype=torch.bool, device="cuda")
+        for d in range(3):
+            inside &= (f[d] - f[d].round()).abs() > edge[d]
+        at = [f[d].floor().long().clamp(0, grid[d] - 1) for d in range(3)]
+        want = (at[2] * grid[1] + at[1]) * grid[0] + at[0]
+        assert torch.equal(cell[inside], want[inside])
+        ids = torch.argsort(cell, stable=True) + 1
+        assert torch.equal(ws.particle_ids_sorted().long(), ids)
+        counts = torch.bincount(cell, minlength=ws.ncell)
+        off = torch.cat((torch.zeros(1, dtype=torch.long, device="cuda"), counts.cumsum(0))) + 1
+        assert torch.equal(ws.cell_offsets().long(), off)
+
+    ws.update(X, Y, Z, None)
+    s = ws.state()
+    assert s[6] == 1 and s[10] == 1 and s[8] == int(ws.counts().max())
+    check()
+    assert (s[1], s[7]) == (1, 1)
+    ws.update(X, Y, Z, None)
+    s = ws.state()
+    assert (s[0], s[6], s[7]) == (0, 2, 1)
+    X.copy_(torch.where(X > 0, X - 1.5, X + 1.5))
+    ws.update(X, Y, Z, None)
+    s = ws.state()
+    # for the displacement; where the moved halves now overlap in too many neighbours, it is refused
+    fits = int(ws.counts().max()) <= ws.cap
+    assert (s[6], s[9], s[10]) == (3, 2, 2) and (s[1], s[7]) == ((1, 2) if fits else (0, 1))
+    check()
