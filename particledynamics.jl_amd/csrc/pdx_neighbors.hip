@@ -1075,10 +1075,8 @@ int enqueue_decide_build(pdx_nl_t nl, hipStream_t st) {
     bool stage = false;
     if (const char *v = std::getenv("PDX_ROW_STAGE")) stage = std::atoi(v) != 0;
     // the cell-staged build (k_rows_cells, PDX_ROW_CELLS=1): at 486 400 ions (8 000 cells, one
-    // workgroup each) 1.06-1.09 ms against 1.12 ms for k_rows in spatial storage order and 1.33
-    // against 1.55 ms in lattice order, but on the checks without rebuild its LDS-holding
-    // workgroups cost 10 us against 5 us, so spatially ordered storage (ForceEngine.reorder)
-    // keeps k_rows; the LDS-staged row write (PDX_ROW_STAGE=1) is a k_rows option
+    // workgroup each) 1.06-1.09 ms against 1.12 ms for k_rows in spatial storage order, 1.33 against
+    // 1.55 ms in lattice order; a whole rebuild with k_rows_masks takes 1.02 ms, with k_rows 1.22
     bool cells = false;
     if (const char *v = std::getenv("PDX_ROW_CELLS")) cells = std::atoi(v) != 0;
     if (stage) cells = false;
