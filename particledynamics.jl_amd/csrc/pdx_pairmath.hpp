@@ -106,6 +106,8 @@ __device__ __forceinline__ void pair_terms(const A &a, const float (&pe)[NP], co
 // pair_terms with the masks on the factors (1/r, (sigma/r)^6, the charge product) instead of the
 // finished terms, so that force and energy share them, and the Coulomb terms joined by fused steps:
 // about seven instructions fewer per visit with energies, equal to pair_terms up to FP32 rounding.
+// The polynomials' argument stops at the end of the fit: far beyond it (a list radius of several
+// real-space cutoffs) they would overflow, and a masked charge product times infinity is no zero.
 // pe[0] carries the cutoff energy shift (-ceshift). A: the fields of pair_terms.
 template <int MODEL, bool COUL, bool ENERGY, int NP, typename A>
 __device__ __forceinline__ void pair_terms_joint(const A &a, const float (&pe)[NP], const float (&pf)[NP], float cqi,
@@ -139,7 +141,7 @@ __device__ __forceinline__ void pair_terms_joint(const A &a, const float (&pe)[N
     if (ENERGY) u = in ? 0.5f * a.eps * xx * xx : 0.f;
   }
   if (COUL) {
-    const float x = fmaf(r2, a.csx, -1.0f);
+    const float x = fminf(fmaf(r2, a.csx, -1.0f), 1.0f);
     const float cq = (pos & (r2 < a.crc2)) ? cqi * qj : 0.f;
     f = fmaf(cq, fmaf(rinv, i2, -horner<NP>(pf, x)), f);
     if (ENERGY) u = fmaf(cq, rinv + horner<NP>(pe, x), u);

@@ -193,3 +193,46 @@ def test_cell_traversal_restrictions(cuda):
     x = torch.zeros(8, device="cuda")
     with pytest.raises(pdx.ArgumentError):
         p.compute(nl, x, x, x, energy=False)
+
+
+@pytest.mark.parametrize("lanes", [0, 1, 4, 64, -4])
+def test_entries_far_beyond_the_real_cutoff(cuda, lanes):
+    """Row entries at up to 6.8 real-space cutoffs (a long LJ cutoff beside a short, tight Coulomb one, whose
+    polynomials overflow there): energy and forces-only launches give the same finite forces."""
+    import torch
+    n, L, rlj, rc, skin = 900, 9.0, 3.0, 0.5, 0.4
+    g = np.stack(np.meshgrid(*(np.arange(10),) * 3, indexing="ij"), -1).reshape(-1, 3)[:n]
+    rng = np.random.default_rng(5)
+    P = ((g + 0.5) * 0.9 - L / 2 + rng.uniform(-0.25, 0.25, (n, 3))).astype(np.float32)
+    q = np.where(np.arange(n) % 2, 1.0, -1.0).astype(np.float32)
+    X, Y, Z, Q = (dev(np.ascontiguousarray(a)) for a in (P[:, 0], P[:, 1], P[:, 2], q))
+    ws = pdx.DeviceNeighborWorkspace(n, (L,) * 3, rlj, skin, 400, allpairs=True)
+    ws.update(X, Y, Z, Q)
+    eps, sig, alpha = 1.0, 0.3, 12.0
+    pf = pdx.PairForce(pdx.LennardJones(eps, sig, rlj), coulomb=pdx.RealSpaceCoulomb(1.0, rc, alpha), lanes=lanes)
+    f, g = ([torch.full((n,), 7.0, device="cuda") for _ in range(3)] for _ in range(2))
+    E = torch.full((n,), 7.0, device="cuda")
+    V = torch.full((6, n), 7.0, device="cuda")
+    tot = torch.zeros(7, dtype=torch.float64, device="cuda")
+    pf.compute(ws, *f, E, V, tot, energy=True)
+    pf.compute(ws, *g, energy=False)
+    ws.status()
+    assert torch.isfinite(torch.cat([*f, *g, E, V.flatten(), tot.float()])).all()
+    d = P[:, None, :].astype(np.float64) - P[None, :, :]
+    d -= L * np.round(d / L)
+    r2 = (d ** 2).sum(-1)
+    np.fill_diagonal(r2, np.inf)
+    s6 = np.where(r2 < rlj ** 2, (sig ** 2 / r2) ** 3, 0.0)
+    r = np.sqrt(r2)
+    erfc = np.vectorize(math.erfc)
+    near = r < rc
+    coul = np.zeros_like(r)
+    coul[near] = erfc(alpha * r[near]) / r[near] + 2 * alpha / math.sqrt(math.pi) * np.exp(-(alpha * r[near]) ** 2)
+    assert near.any() and (r2[np.isfinite(r2)] < (rlj + skin) ** 2).any()
+    size = (24 * eps * (2 * s6 * s6 + s6) + coul) / r  # |f| of each pair
+    # two FP32 sums of at most 400 terms; a term's own rounding is below 64 ulps (the twelfth power of an
+    # inverse root of one ulp, and the difference of 1/r^3 and the polynomial, both under 1/r^3)
+    size[near] += 2 / r[near] ** 2
+    bound = 2 * (400 + 64) * 6e-8 * size.sum(1)
+    dF = (torch.stack(f, 1) - torch.stack(g, 1)).double().cpu().numpy()
+    assert (np.abs(dF).max(1) <= bound).all()
