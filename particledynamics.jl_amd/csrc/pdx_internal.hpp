@@ -319,6 +319,7 @@ struct pdx_pair_s {
   float pe[24] = {0}, pf[24] = {0};
   double fit_err_e = 0, fit_err_f = 0;
   int lanes = 4;
+  bool wide = false;  // 64-bit row addresses at any size (pdx_test_pair_wide)
   int accumulate = PDX_ACC_FP32;      // force / energy / virial accumulator of the row sums
   int traversal = PDX_TRAVERSAL_ROWS;  // rows of the list, or the list's cells directly
   struct pdx_bonds_s *bonds = nullptr;  // FENE bonds folded into the same per-particle sums
@@ -395,3 +396,6 @@ struct pdx_mesh_s {
   pdx::DevBuf<unsigned long long> tile_blocks;
   size_t tile_block_entries = 0;
 };
+
+// For tests: the row walk with 64-bit addresses, which only lists beyond 32-bit offsets take, at any size.
+extern "C" int pdx_test_pair_wide(pdx_pair_t p, int32_t on);

@@ -4,6 +4,7 @@
 
 #include "pdx_internal.hpp"
 #include "pdx_pairmath.hpp"
+#include "pdx_rowwalk.hpp"
 
 namespace pdx {
 namespace pairk {
@@ -92,7 +93,7 @@ __device__ __forceinline__ void pair_epilogue(const PairArgs &a, bool owner, int
 // pair terms; 486 400 ions, 4 lanes: 258 -> 242 us, 64 000 ions: 37 -> 32 us). Forces only it is 49,
 // fewer than the gather's share of the L1 (75 clocks per wave and visit), which then bounds the walk
 // (224 -> 220 us).
-// Lists beyond the 32-bit offsets (G N >= 2^28 even with one lane: WIDE) take 64-bit addresses.
+// Lists beyond the 32-bit offsets even with one lane (walk_shape) take 64-bit addresses: WIDE.
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 constexpr int BUFFER_RAW = 0x00020000;  // word 3 of a raw buffer resource on gfx9
 template <int G, int U, bool WIDE, class VISIT>
@@ -103,7 +104,7 @@ __device__ __forceinline__ void walk_rows(const PairArgs &a, const float4 &pi, i
                                    (fabsf(pi.z) > hz - a.reach));
   const bool seam = __ballot(near_face) != 0;
   // ids are 1-based: the resource starts one particle early
-  const auto prs = __builtin_amdgcn_make_buffer_rsrc((void *)(a.packed - 1), 0, (N + 1) * 16, BUFFER_RAW);
+  const auto prs = __builtin_amdgcn_make_buffer_rsrc((void *)(a.packed - 1), 0, (int)walk_records(N), BUFFER_RAW);
   auto eval = [&](const int (&id)[U]) {
     float4 pj[U];
     int jj[U];
@@ -113,7 +114,7 @@ __device__ __forceinline__ void walk_rows(const PairArgs &a, const float4 &pi, i
       if (WIDE) {
         pj[u] = a.packed[jj[u]];
       } else {
-        const u32x4 w = __builtin_amdgcn_raw_buffer_load_b128(prs, (int)((unsigned)id[u] << 4), 0, 0);
+        const u32x4 w = __builtin_amdgcn_raw_buffer_load_b128(prs, (int)walk_gather(id[u]), 0, 0);
         pj[u] = make_float4(__uint_as_float(w.x), __uint_as_float(w.y), __uint_as_float(w.z), __uint_as_float(w.w));
       }
     }
@@ -133,12 +134,12 @@ __device__ __forceinline__ void walk_rows(const PairArgs &a, const float4 &pi, i
   const int32_t *row = a.nbr + i;
   const int full = WIDE ? 0 : __builtin_amdgcn_readfirstlane(wave_min(n) / (U * G));
   const int its = __builtin_amdgcn_readfirstlane((wave_max(n) + U * G - 1) / (U * G));
-  const int vo = (int)(((unsigned)lane * (unsigned)N + (unsigned)i) * 4u);
+  const int vo = (int)walk_lane(lane, N, i);
   auto load = [&](int k, int (&id)[U]) {
     if (k < full) {
       const auto rrs = __builtin_amdgcn_make_buffer_rsrc((void *)(a.nbr + (size_t)k * (U * G) * N), 0, -1, BUFFER_RAW);
 #pragma unroll
-      for (int u = 0; u < U; ++u) id[u] = (int)__builtin_amdgcn_raw_buffer_load_b32(rrs, vo, u * G * N * 4, 0);
+      for (int u = 0; u < U; ++u) id[u] = (int)__builtin_amdgcn_raw_buffer_load_b32(rrs, vo, (int)walk_step(u, G, N), 0);
     } else {
 #pragma unroll
       for (int u = 0; u < U; ++u) {
@@ -193,7 +194,7 @@ __global__ __launch_bounds__(TPB, ENERGY ? 6 : 8) void k_pair(const PairArgs a) 
     // typed models: i's diameter, or its type's row of the table
     const float ci = MIXED ? a.sigp[ic] : 0.f;
     const int ti = (TYPED && !MIXED) ? (a.typ[ic] - 1) * a.ntypes : 0;
-    constexpr int U = 4;
+    constexpr int U = WALK_U;
     walk_rows<G, U, WIDE>(a, pi, ic, lane, active, active ? a.counts[ic] : 0, hx, hy, hz, Lx, Ly, Lz,
                     [&](const int (&jj)[U], const float4 (&pj)[U], const float (&ddx)[U], const float (&ddy)[U],
                         const float (&ddz)[U]) {
@@ -631,7 +632,7 @@ __global__ __launch_bounds__(TPB, ACC == PDX_ACC_FP32 ? 6 : 1) void k_pair_acc(c
 #pragma unroll
       for (int k = 0; k < 4; ++k) bp[k] = k < nbx ? a.bpart[bx0 + k] : -1;
     }
-    constexpr int U = 4;
+    constexpr int U = WALK_U;
     walk_rows<G, U, WIDE>(a, pi, ic, lane, active, n, hx, hy, hz, Lx, Ly, Lz,
                     [&](const int (&jj)[U], const float4 (&)[U], const float (&ddx)[U], const float (&ddy)[U],
                         const float (&ddz)[U]) {

@@ -280,9 +280,8 @@ int pair_forces_impl(pdx_pair_t p, pdx_nl_t nl, float *fx, float *fy, float *fz,
     if (!acc_path && rows >= 32.0) G = std::max(G, 4);
   }
   if (acc_path) G = std::min(G, 8);
-  // the row walk's 32-bit offsets: fewer lanes for lists that would exceed them
-  while (G > 1 && (int64_t)G * N >= (1ll << 28)) G >>= 1;
-  const int shape = G == 1 && N >= (1 << 28) ? 0 : G;  // 0: one lane with 64-bit addresses
+  const int shape = p->wide && G > 0 ? 0 : walk_shape(G, N);  // 0: one lane with 64-bit addresses
+  if (shape >= 0) G = std::max(shape, 1);
   const int blocks = cells ? nl->ncell
                            : (G < 0 ? (N + WAVE - 1) / WAVE : (int)(((int64_t)N * G + TPB - 1) / TPB));
   double *partial = fixed_partial;
@@ -652,5 +651,11 @@ extern "C" int pdx_pair_set_traversal(pdx_pair_t p, int32_t mode) {
   if (mode != PDX_TRAVERSAL_ROWS && mode != PDX_TRAVERSAL_CELLS)
     return fail(PDX_ERR_ARGUMENT, "traversal must be PDX_TRAVERSAL_ROWS or PDX_TRAVERSAL_CELLS");
   p->traversal = mode;
+  return PDX_OK;
+}
+
+extern "C" int pdx_test_pair_wide(pdx_pair_t p, int32_t on) {
+  if (!p) return fail(PDX_ERR_ARGUMENT, "null pair model");
+  p->wide = on != 0;
   return PDX_OK;
 }
