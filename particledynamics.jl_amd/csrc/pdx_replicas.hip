@@ -56,6 +56,12 @@ __device__ __forceinline__ float wrap_centred(float x, float L) {
   return x;
 }
 
+// The image in the box of a coordinate outside it: a caller's, or of an atom that crossed more than the
+// box in one step, which wrap_centred shifts once. Cells and pair distances are taken from it.
+__device__ __forceinline__ float into_box(float x, float halfL, float L) {
+  return x >= -halfL && x <= halfL ? x : x - L * floorf((x + halfL) / L);
+}
+
 // Force factor f (force on i = f d) and energy u of one pair (same arithmetic as the ELL
 // pair kernel: 24e(2s^12 - s^6)/r^2; u = 4e(s^12 - s^6) - u_c, or + e for WCA).
 __device__ __forceinline__ void lj_terms(const Rep &R, float r2, float &f, float &u) {
@@ -132,8 +138,9 @@ __device__ __forceinline__ void atom_forces(const Rep &R, const float4 *spos, co
       const float rem = fmaf(-dy, dy, remz);
       if (!(rem > 0.f)) continue;
       const float xr = __builtin_amdgcn_sqrtf(rem) + R.slack;  // (its ulp is within the slack)
-      const int x0 = max((int)floorf((ux - xr) * R.cinv[0]), cx - S);
-      const int x1 = min((int)floorf((ux + xr) * R.cinv[0]), cx + S);
+      // (both include the atom's own cell, whatever its coordinate: no cell outside the table is read)
+      const int x0 = min(max((int)floorf((ux - xr) * R.cinv[0]), cx - S), cx);
+      const int x1 = max(min((int)floorf((ux + xr) * R.cinv[0]), cx + S), cx);
       int y2 = cy + oy;
       float py = p.y;
       if (y2 < 0) { y2 += ny; py += R.L[1]; } else if (y2 >= ny) { y2 -= ny; py -= R.L[1]; }
@@ -171,7 +178,8 @@ __global__ __launch_bounds__(BS) void k_replicas(const Rep *__restrict__ reps, c
   char *base0 = reinterpret_cast<char *>(smem) + reg0;
   unsigned short *cst = reinterpret_cast<unsigned short *>(base0);     // cell starts
   unsigned *cnt = reinterpret_cast<unsigned *>(base0 + reg1);          // next counts, two 16-bit cells a word
-  int *wsum = reinterpret_cast<int *>(base0 + reg1 + reg2);
+  int *wsum = reinterpret_cast<int *>(base0 + reg1 + reg2);  // 16 wave sums
+  int *outside = wsum + 16;                                  // some atom's coordinates are an image of its own
   double *red = reinterpret_cast<double *>(base0 + reg1 + reg2 + 128);
 
   const int rid = order[blockIdx.x];
@@ -187,6 +195,9 @@ __global__ __launch_bounds__(BS) void k_replicas(const Rep *__restrict__ reps, c
   // the atom's cell for the next scatter: its rank among the cell's atoms so far
   auto bin = [&](int g, float px, float py, float pz) {
     if (allpairs) return;
+    px = into_box(px, R.halfL[0], R.L[0]);
+    py = into_box(py, R.halfL[1], R.L[1]);
+    pz = into_box(pz, R.halfL[2], R.L[2]);
     const int cell = (cell_coord(pz, R.halfL[2], R.cinv[2], R.nc[2]) * R.nc[1] +
                       cell_coord(py, R.halfL[1], R.cinv[1], R.nc[1])) * R.nc[0] +
                      cell_coord(px, R.halfL[0], R.cinv[0], R.nc[0]);
@@ -235,7 +246,10 @@ __global__ __launch_bounds__(BS) void k_replicas(const Rep *__restrict__ reps, c
         cst[k] = (unsigned short)base;
         base += count(k);
       }
-      if (t == 0) cst[ncell] = (unsigned short)n;
+      if (t == 0) {
+        cst[ncell] = (unsigned short)n;
+        *outside = 0;
+      }
       __syncthreads();
       // ---- C: scatter into cell order; the counts are cleared for E
       for (int k = t; k < (ncell + 1) / 2; k += BS) cnt[k] = 0u;
@@ -243,7 +257,11 @@ __global__ __launch_bounds__(BS) void k_replicas(const Rep *__restrict__ reps, c
         const int g = off + i;
         const unsigned kk = (unsigned)key[g];
         const int slot = cst[kk & 0xffffu] + (int)(kk >> 16);
-        spos[slot] = make_float4(x[g], y[g], z[g], __int_as_float(i));
+        const float px = x[g], py = y[g], pz = z[g];
+        const float4 p = make_float4(into_box(px, R.halfL[0], R.L[0]), into_box(py, R.halfL[1], R.L[1]),
+                                     into_box(pz, R.halfL[2], R.L[2]), __int_as_float(i));
+        if (!(p.x == px && p.y == py && p.z == pz)) *outside = 1;
+        spos[slot] = p;
       }
       __syncthreads();
       // ---- D: atom-id order inside every cell
@@ -266,6 +284,7 @@ __global__ __launch_bounds__(BS) void k_replicas(const Rep *__restrict__ reps, c
     __syncthreads();
     // ---- E: forces, the closing kick, and the next step's kick-drift and cell count
     const bool acc = last && energy;
+    const bool images = !allpairs && *outside != 0;
     for (int q = t; q < n * G; q += BS) {
       const int s = q / G, sub = q - s * G;
       const float4 p = spos[s];
@@ -289,6 +308,8 @@ __global__ __launch_bounds__(BS) void k_replicas(const Rep *__restrict__ reps, c
         fx[g] = ax; fy[g] = ay; fz[g] = az;
         if (integrate) { vx[g] = ux; vy[g] = uy; vz[g] = uz; }
         if (acc) ke += 0.5 * (double)mass * ((double)ux * ux + (double)uy * uy + (double)uz * uz);
+      } else if (images) {
+        kick_drift(g, fmaf(c, ax, ux), fmaf(c, ay, uy), fmaf(c, az, uz), x[g], y[g], z[g]);
       } else {
         kick_drift(g, fmaf(c, ax, ux), fmaf(c, ay, uy), fmaf(c, az, uz), p.x, p.y, p.z);
       }

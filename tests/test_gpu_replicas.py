@@ -195,3 +195,83 @@ def test_forces_at_the_size_steps(cuda, n, model, aspect):
     assert abs(out[0] - d["energy"].sum()) <= 1e-5 * max(np.abs(d["energy"]).sum(), 1e-30)
     assert abs(out[2] - d["virial"][:, :3].sum()) <= 1e-5 * max(np.abs(d["virial"]).sum(), 1e-30)
     assert out[3] == n
+
+
+@pytest.mark.parametrize("stencil", [0, 1, 2])
+def test_atoms_outside_the_box(cuda, stencil):
+    """Coordinates that are images outside [-L/2, L/2): forces, energies and virials are those of the
+    atoms in the box, and the first drift goes on from the coordinates as given."""
+    import torch
+    rng = np.random.default_rng(4)
+    boxes = [(9.0, 10.0, 11.0), (9.5, 9.0, 8.75), (26.0, 25.0, 24.0)]
+    specs, P, S = [], [], []
+    for k, box in enumerate(boxes):
+        n = (700, 520, 8192)[k]
+        m = int(np.ceil(n ** (1 / 3)))
+        g = np.stack(np.meshgrid(*(np.arange(m),) * 3, indexing="ij"), -1).reshape(-1, 3)[rng.permutation(m ** 3)[:n]]
+        L = np.array(box)
+        X = ((g + 0.5 + 0.08 * rng.standard_normal(g.shape)) / m - 0.5) * L
+        X = np.clip(X, -L / 2 + 0.01, L / 2 - 0.01)
+        X = np.round(X * 2.0 ** 14) / 2.0 ** 14  # shifts by a box are then exact in FP32
+        shift = np.zeros_like(X)
+        some = rng.permutation(n)[:n // 4]
+        shift[some] = rng.integers(-2, 3, (len(some), 3))
+        for d in range(3):  # a little outside: an atom next to a face as the image across the other one
+            shift[X[:, d] > L[d] / 2 - 0.3, d] = -1
+        specs.append({"model": ("lj", "wca", "lj")[k], "n": n, "box": box, "cutoff": 2.5})
+        P.append(X)
+        S.append(shift * L)
+    X, S = np.concatenate(P), np.concatenate(S)
+    v = 0.3 * rng.standard_normal(X.shape)
+
+    def state(X):
+        return replicas.device_state(dict(x=X[:, 0], y=X[:, 1], z=X[:, 2], vx=v[:, 0], vy=v[:, 1], vz=v[:, 2]))
+    rb = pdx.ReplicaBatch(specs, stencil=stencil)
+    a, b = state(X), state(X + S)
+    assert (np.abs(S) > 0).any() and np.array_equal((X + S).astype(np.float32).astype(np.float64), X + S)
+    ea, eb = rb.forces(a), rb.forces(b)
+    for k in ("fx", "fy", "fz"):
+        assert torch.equal(a[k], b[k]), k
+        assert torch.isfinite(a[k]).all() and a[k].abs().max() > 1
+    assert torch.equal(ea, eb)
+    # dt = 0: the step is the wrap alone, which shifts by one box at most
+    c = state(X + S)
+    rb.run(c, 1, dt=0.0, forces_valid=False)
+    L = np.repeat(np.array(boxes), [s["n"] for s in specs], axis=0).astype(np.float32)
+    Y = (X + S).astype(np.float32)
+    Y = np.where(Y >= L / 2, Y - L, Y)
+    Y = np.where(Y < -L / 2, Y + L, Y)
+    for d, k in enumerate("xyz"):
+        assert np.array_equal(c[k].cpu().numpy(), Y[:, d]), k
+
+
+def test_coordinates_without_a_cell(cuda):
+    """Huge coordinates stay inside the tables: the other atoms' forces are those of a box without these
+    atoms. Infinite and undefined ones reach no other replica."""
+    import torch
+    b = _small_batch(seed=2, nrep=2, n_range=(600, 600))
+    huge = {5: 3e38, 17: -3e38, 77: 1e20, 601: -1e20, 700: 1e9}
+    rb = pdx.ReplicaBatch(b["specs"])
+    good = replicas.device_state(b)
+    st = replicas.clone_state(good)
+    for i, x in huge.items():
+        st["x"][i] = x
+        st["y"][i] = x
+    rb.forces(st)
+    for k in range(2):
+        lo, hi = int(rb.offsets[k]), int(rb.offsets[k + 1])
+        keep = [i for i in range(lo, hi) if i not in huge]
+        one = pdx.ReplicaBatch([dict(b["specs"][k], n=len(keep))])
+        s1 = {a: t[keep].contiguous() for a, t in good.items()}
+        one.forces(s1)
+        for a in ("fx", "fy", "fz"):
+            # the same pairs, in rows that the missing atoms pair differently: rounding of ~60 terms
+            d = (s1[a] - st[a][keep]).abs().max()
+            assert torch.isfinite(st[a][keep]).all() and d <= 1e-4 * s1[a].abs().max(), (k, a)
+    rb.forces(good)
+    st = replicas.clone_state(good)
+    for i, x in {5: np.inf, 17: -np.inf, 77: np.nan}.items():
+        st["x"][i] = x
+    rb.forces(st)
+    for a in ("fx", "fy", "fz"):
+        assert torch.equal(st[a][600:], good[a][600:]), a
