@@ -56,10 +56,13 @@ __device__ __forceinline__ float wrap_centred(float x, float L) {
   return x;
 }
 
-// The image in the box of a coordinate outside it: a caller's, or of an atom that crossed more than the
-// box in one step, which wrap_centred shifts once. Cells and pair distances are taken from it.
+// Coordinates outside the box are a caller's, or of an atom that crossed more than the box in one step,
+// which wrap_centred shifts once. Cells and pair distances are then taken from the image in the box.
+__device__ __forceinline__ bool outside_box(const Rep &R, float x, float y, float z) {
+  return !(fabsf(x) <= R.halfL[0] && fabsf(y) <= R.halfL[1] && fabsf(z) <= R.halfL[2]);
+}
 __device__ __forceinline__ float into_box(float x, float halfL, float L) {
-  return x >= -halfL && x <= halfL ? x : x - L * floorf((x + halfL) / L);
+  return fabsf(x) <= halfL ? x : x - L * floorf((x + halfL) / L);
 }
 
 // Force factor f (force on i = f d) and energy u of one pair (same arithmetic as the ELL
@@ -119,7 +122,9 @@ __device__ __forceinline__ void atom_forces(const Rep &R, const float4 *spos, co
   const int cx = cell_coord(p.x, R.halfL[0], R.cinv[0], nx);
   const int cy = cell_coord(p.y, R.halfL[1], R.cinv[1], ny);
   const int cz = cell_coord(p.z, R.halfL[2], R.cinv[2], nz);
-  const float ux = p.x + R.halfL[0];
+  // 0 <= ux <= L whatever the coordinate (one that no shift brings into the box, NaN): with it every
+  // row has x0 <= nx - 1 and x1 >= 0, and no cell outside the table is read
+  const float ux = __builtin_amdgcn_fmed3f(p.x + R.halfL[0], 0.f, R.L[0]);
   int r = 0;
   for (int oz = -S; oz <= S; ++oz) {
     // a row's distance from the atom in z and y, less a slack that covers the rounding of the edges
@@ -138,9 +143,8 @@ __device__ __forceinline__ void atom_forces(const Rep &R, const float4 *spos, co
       const float rem = fmaf(-dy, dy, remz);
       if (!(rem > 0.f)) continue;
       const float xr = __builtin_amdgcn_sqrtf(rem) + R.slack;  // (its ulp is within the slack)
-      // (both include the atom's own cell, whatever its coordinate: no cell outside the table is read)
-      const int x0 = min(max((int)floorf((ux - xr) * R.cinv[0]), cx - S), cx);
-      const int x1 = max(min((int)floorf((ux + xr) * R.cinv[0]), cx + S), cx);
+      const int x0 = max((int)floorf((ux - xr) * R.cinv[0]), cx - S);
+      const int x1 = min((int)floorf((ux + xr) * R.cinv[0]), cx + S);
       int y2 = cy + oy;
       float py = p.y;
       if (y2 < 0) { y2 += ny; py += R.L[1]; } else if (y2 >= ny) { y2 -= ny; py -= R.L[1]; }
@@ -179,7 +183,7 @@ __global__ __launch_bounds__(BS) void k_replicas(const Rep *__restrict__ reps, c
   unsigned short *cst = reinterpret_cast<unsigned short *>(base0);     // cell starts
   unsigned *cnt = reinterpret_cast<unsigned *>(base0 + reg1);          // next counts, two 16-bit cells a word
   int *wsum = reinterpret_cast<int *>(base0 + reg1 + reg2);  // 16 wave sums
-  int *outside = wsum + 16;                                  // some atom's coordinates are an image of its own
+  int *outside = wsum + 16;                                  // an atom of the coming step is outside the box
   double *red = reinterpret_cast<double *>(base0 + reg1 + reg2 + 128);
 
   const int rid = order[blockIdx.x];
@@ -195,9 +199,12 @@ __global__ __launch_bounds__(BS) void k_replicas(const Rep *__restrict__ reps, c
   // the atom's cell for the next scatter: its rank among the cell's atoms so far
   auto bin = [&](int g, float px, float py, float pz) {
     if (allpairs) return;
-    px = into_box(px, R.halfL[0], R.L[0]);
-    py = into_box(py, R.halfL[1], R.L[1]);
-    pz = into_box(pz, R.halfL[2], R.L[2]);
+    if (outside_box(R, px, py, pz)) {
+      px = into_box(px, R.halfL[0], R.L[0]);
+      py = into_box(py, R.halfL[1], R.L[1]);
+      pz = into_box(pz, R.halfL[2], R.L[2]);
+      *outside = 1;
+    }
     const int cell = (cell_coord(pz, R.halfL[2], R.cinv[2], R.nc[2]) * R.nc[1] +
                       cell_coord(py, R.halfL[1], R.cinv[1], R.nc[1])) * R.nc[0] +
                      cell_coord(px, R.halfL[0], R.cinv[0], R.nc[0]);
@@ -216,6 +223,7 @@ __global__ __launch_bounds__(BS) void k_replicas(const Rep *__restrict__ reps, c
   };
 
   for (int k = t; k < (ncell + 1) / 2; k += BS) cnt[k] = 0u;
+  if (t == 0) *outside = 0;
   __syncthreads();
   for (int i = t; i < n; i += BS) {
     const int g = off + i;
@@ -226,6 +234,7 @@ __global__ __launch_bounds__(BS) void k_replicas(const Rep *__restrict__ reps, c
   for (int step = first_force ? 0 : 1; step <= nsteps; ++step) {
     const bool integrate = step > 0;
     const bool last = step == nsteps;
+    bool images = false;  // some atom's coordinates are not its slot's
     if (!allpairs) {
       // ---- B: exclusive scan of the counts (contiguous chunk per thread, wave scans)
       const int k0 = min(t * chunk, ncell), k1 = min(k0 + chunk, ncell);
@@ -246,24 +255,25 @@ __global__ __launch_bounds__(BS) void k_replicas(const Rep *__restrict__ reps, c
         cst[k] = (unsigned short)base;
         base += count(k);
       }
-      if (t == 0) {
-        cst[ncell] = (unsigned short)n;
-        *outside = 0;
-      }
+      if (t == 0) cst[ncell] = (unsigned short)n;
       __syncthreads();
+      images = *outside != 0;
       // ---- C: scatter into cell order; the counts are cleared for E
       for (int k = t; k < (ncell + 1) / 2; k += BS) cnt[k] = 0u;
       for (int i = t; i < n; i += BS) {
         const int g = off + i;
         const unsigned kk = (unsigned)key[g];
         const int slot = cst[kk & 0xffffu] + (int)(kk >> 16);
-        const float px = x[g], py = y[g], pz = z[g];
-        const float4 p = make_float4(into_box(px, R.halfL[0], R.L[0]), into_box(py, R.halfL[1], R.L[1]),
-                                     into_box(pz, R.halfL[2], R.L[2]), __int_as_float(i));
-        if (!(p.x == px && p.y == py && p.z == pz)) *outside = 1;
+        float4 p = make_float4(x[g], y[g], z[g], __int_as_float(i));
+        if (images) {
+          p.x = into_box(p.x, R.halfL[0], R.L[0]);
+          p.y = into_box(p.y, R.halfL[1], R.L[1]);
+          p.z = into_box(p.z, R.halfL[2], R.L[2]);
+        }
         spos[slot] = p;
       }
       __syncthreads();
+      if (t == 0) *outside = 0;
       // ---- D: atom-id order inside every cell
       for (int cell = t; cell < ncell; cell += BS) {
         const int b = cst[cell], e = cst[cell + 1];
@@ -284,7 +294,6 @@ __global__ __launch_bounds__(BS) void k_replicas(const Rep *__restrict__ reps, c
     __syncthreads();
     // ---- E: forces, the closing kick, and the next step's kick-drift and cell count
     const bool acc = last && energy;
-    const bool images = !allpairs && *outside != 0;
     for (int q = t; q < n * G; q += BS) {
       const int s = q / G, sub = q - s * G;
       const float4 p = spos[s];
