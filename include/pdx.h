@@ -583,8 +583,8 @@ typedef struct {
 
 typedef struct pdx_rep_s *pdx_rep_t;
 /* Replica set: atoms of replica k occupy [offset_k, offset_k + n_k) of the concatenated SoA
- * arrays (offsets = prefix sums of n). block: workgroup size 256 / 512 / 1024 (0: 1024);
- * stencil: cells per cutoff, 1 (27 cells of side >= rc) or 2 (125 cells of side >= rc/2)
+ * arrays (offsets = prefix sums of n). block: workgroup size 256 / 512 / 1024
+ * (0: by the replicas' sizes); stencil: cells per cutoff, 1 (27 cells of side >= rc) or 2 (125 cells of side >= rc/2)
  * (0: per replica, 2 where the finer cells fit the table); boxes with fewer than three cells
  * of side rc use all pairs, and so do those too small for an explicit stencil. */
 int pdx_replicas_create(int32_t nrep, const pdx_replica_spec *specs, int32_t block, int32_t stencil,

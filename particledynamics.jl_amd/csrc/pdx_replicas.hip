@@ -19,7 +19,7 @@
 // a stencil is walked as (2S+1)^2 rows of cells, contiguous in LDS; a row further than rc is left
 // out and the others are cut to the cells a sphere of rc reaches; a row's image shift is subtracted
 // from the atom once instead of testing every pair. 512 boxes of 256..8192 atoms, 20 steps: 31.0 ms
-// with 27-cell stencils, a separate kick-drift pass and 512 threads, 8.6 ms now (0.43 ms a step).
+// with 27-cell stencils, a separate kick-drift pass and 512 threads, 8.5 ms now (0.42 ms a step).
 #include "pdx_internal.hpp"
 
 #include <algorithm>
@@ -89,12 +89,14 @@ __device__ __forceinline__ double block_sum(double v, double *red) {
   return s;
 }
 
-// Lanes per atom of the force phase: small replicas would leave most of the workgroup idle. A
-// function of n alone, as the lanes' partial sums are part of the replica's arithmetic.
-__host__ __device__ inline int atom_lanes(int n) { return n <= 512 ? 4 : (n <= 1024 ? 2 : 1); }
+// Lanes per atom of the force phase: two share the atoms of a small box on all pairs (16 boxes of 200
+// atoms, 10 steps: 316 -> 177 us), where each lane's half is as long. The rows of a stencil are cut to a
+// sphere and share badly: with two and four lanes 16 boxes of 700 atoms took 785 and 1 256 us, with one
+// 502. A function of the replica alone, as the lanes' partial sums are part of its arithmetic.
+__host__ __device__ inline int atom_lanes(const Rep &R) { return R.S == 0 && R.n <= 256 ? 2 : 1; }
 
-// Forces on the atom at p (slot s): its share (rows sub, sub + G, ...) of the stencil's rows of cells,
-// in row order, every row in x order. ENERGY also sums the pair energies and r.F.
+// Forces on the atom at p (slot s): every G-th atom from sub on of a box on all pairs, else the stencil's
+// rows of cells in row order, every row in x order. ENERGY also sums the pair energies and r.F.
 template <bool ENERGY>
 __device__ __forceinline__ void atom_forces(const Rep &R, const float4 *spos, const unsigned short *cst, int n,
                                             const float4 &p, int s, int sub, int G, float &ax, float &ay, float &az,
@@ -125,7 +127,6 @@ __device__ __forceinline__ void atom_forces(const Rep &R, const float4 *spos, co
   // 0 <= ux <= L whatever the coordinate (one that no shift brings into the box, NaN): with it every
   // row has x0 <= nx - 1 and x1 >= 0, and no cell outside the table is read
   const float ux = __builtin_amdgcn_fmed3f(p.x + R.halfL[0], 0.f, R.L[0]);
-  int r = 0;
   for (int oz = -S; oz <= S; ++oz) {
     // a row's distance from the atom in z and y, less a slack that covers the rounding of the edges
     const float gz = (float)(cz + oz) * R.cw[2] - R.halfL[2];
@@ -135,8 +136,7 @@ __device__ __forceinline__ void atom_forces(const Rep &R, const float4 *spos, co
     int z2 = cz + oz;
     float pz = p.z;
     if (z2 < 0) { z2 += nz; pz += R.L[2]; } else if (z2 >= nz) { z2 -= nz; pz -= R.L[2]; }
-    for (int oy = -S; oy <= S; ++oy, ++r) {
-      if (G > 1 && (r & (G - 1)) != sub) continue;
+    for (int oy = -S; oy <= S; ++oy) {
       const float gy = (float)(cy + oy) * R.cw[1] - R.halfL[1];
       float dy = oy > 0 ? gy - p.y : (oy < 0 ? p.y - (gy + R.cw[1]) : 0.f);
       dy = fmaxf(dy - R.slack, 0.f);
@@ -193,7 +193,7 @@ __global__ __launch_bounds__(BS) void k_replicas(const Rep *__restrict__ reps, c
   const bool allpairs = R.S == 0;
   const int ncell = allpairs ? 0 : R.nc[0] * R.nc[1] * R.nc[2];
   const int chunk = (ncell + BS - 1) / BS;
-  const int G = atom_lanes(n);
+  const int G = atom_lanes(R);
   double pe = 0.0, ke = 0.0, vir = 0.0;
 
   // the atom's cell for the next scatter: its rank among the cell's atoms so far
@@ -347,14 +347,32 @@ struct pdx_rep_s {
   std::vector<Rep> host;
   std::vector<int64_t> offsets;
   int nrep = 0, nmax = 0, ncmax = 0, block = 1024, stencil = 0, nallpairs = 0;
+  bool block_given = false;
   int64_t total = 0;
   size_t reg0 = 0, reg1 = 0, reg2 = 0, lds = 0;
-
   DevBuf<Rep> reps;
   DevBuf<int32_t> order, key;
 };
 
 namespace {
+
+// The default workgroup: the smallest that gives every lane of the largest replica's atoms a thread, as
+// idle waves keep other replicas off the CU (4 096 boxes of 64 atoms, 10 steps: 256 / 512 / 1024 threads
+// 0.66 / 1.2 / 2.3 ms; 16 boxes of 700 atoms: 1.10 / 0.72 / 0.50 ms; 512 of 2 048: 2.9 / 2.0 / 2.1 ms).
+// With more than two replicas a CU it is the mean replica's (512 at least beside larger ones): the
+// largest one then shares the time with the others.
+int default_block(const std::vector<Rep> &reps) {
+  int64_t sum = 0;
+  int largest = 0;
+  for (const Rep &R : reps) {
+    const int slots = R.n * atom_lanes(R);
+    largest = std::max(largest, slots);
+    sum += slots;
+  }
+  int slots = largest;
+  if (reps.size() > 512) slots = std::max((int)(sum / (int64_t)reps.size()), largest > 512 ? 512 : 0);
+  return slots <= 256 ? 256 : (slots <= 512 ? 512 : 1024);
+}
 
 // Cell tables for stencil half-width S (1 or 2; 0: per replica, 2 where its finer cells fit the
 // table): cells of side >= rc / S, at least 2S + 1 a
@@ -428,6 +446,7 @@ int layout(pdx_rep_t r, int S) {
     r->nmax = std::max(r->nmax, R.n);
     r->host[k] = R;
   }
+  if (!r->block_given) r->block = default_block(r->host);
   r->reg0 = 16 * (size_t)r->nmax;
   r->reg1 = align16(2 * ((size_t)r->ncmax + 1));
   r->reg2 = align16(2 * ((size_t)r->ncmax + 1));
@@ -476,9 +495,7 @@ extern "C" int pdx_replicas_create(int32_t nrep, const pdx_replica_spec *specs, 
   if (!out || !specs) return fail(PDX_ERR_ARGUMENT, "null argument");
   *out = nullptr;
   if (nrep < 1) return fail(PDX_ERR_ARGUMENT, "at least one replica is required");
-  // 1024 threads: the coordinates of the largest replicas leave room for one workgroup per CU
-  if (block == 0) block = 1024;
-  if (block != 256 && block != 512 && block != 1024) return fail(PDX_ERR_ARGUMENT, "block must be 256, 512 or 1024");
+  if (block != 0 && block != 256 && block != 512 && block != 1024) return fail(PDX_ERR_ARGUMENT, "block must be 256, 512 or 1024");
   if (stencil != 0 && stencil != 1 && stencil != 2) return fail(PDX_ERR_ARGUMENT, "stencil must be 1 or 2");
   int64_t total = 0;
   for (int k = 0; k < nrep; ++k) {
@@ -505,7 +522,8 @@ extern "C" int pdx_replicas_create(int32_t nrep, const pdx_replica_spec *specs, 
   r->offsets[0] = 0;
   for (int k = 0; k < nrep; ++k) r->offsets[k + 1] = r->offsets[k] + specs[k].n;
   r->total = total;
-  r->block = block;
+  r->block_given = block != 0;
+  if (block) r->block = block;
   int rc;
   if ((rc = r->reps.alloc(nrep)) || (rc = r->order.alloc(nrep)) || (rc = r->key.alloc(total)) ||
       (rc = layout(r, stencil))) {
@@ -526,6 +544,7 @@ extern "C" int pdx_replicas_set_launch(pdx_rep_t r, int32_t block, int32_t stenc
   if (block != 256 && block != 512 && block != 1024) return fail(PDX_ERR_ARGUMENT, "block must be 256, 512 or 1024");
   if (stencil != 1 && stencil != 2) return fail(PDX_ERR_ARGUMENT, "stencil must be 1 or 2");
   r->block = block;
+  r->block_given = true;
   return stencil == r->stencil ? PDX_OK : layout(r, stencil);
 }
 

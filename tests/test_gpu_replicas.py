@@ -275,3 +275,33 @@ def test_coordinates_without_a_cell(cuda):
     rb.forces(st)
     for a in ("fx", "fy", "fz"):
         assert torch.equal(st[a][600:], good[a][600:]), a
+
+
+@pytest.mark.parametrize("sizes,copies,block", [((64,), 16, 256), ((64,), 600, 256), ((128, 64), 4, 256), ((200,), 8, 512),
+                                                ((260,), 3, 512), ((700,), 3, 1024), ((64, 700), 300, 512),
+                                                ((64, 700), 100, 1024)])
+def test_default_workgroup(cuda, sizes, copies, block):
+    """The default workgroup has a thread for every lane of the largest replica (two lanes an atom up to
+    256 atoms on all pairs), of the mean one where there are more than two replicas a CU; the replicas'
+    results are those of any other shape."""
+    import torch
+    specs, data = [], []
+    for n in sizes:
+        b = systems.replica_batch(1, seed=n, n_range=(n, n), models=("lj",) if n >= 200 else ("wca",))
+        specs += b["specs"]
+        data.append(b)
+    st = {a: np.tile(np.concatenate([b[a] for b in data]), copies) for a in ("x", "y", "z", "vx", "vy", "vz")}
+    rb = pdx.ReplicaBatch(specs * copies)
+    assert rb.info()["block"] == block
+    a = replicas.device_state(st)
+    rb.forces(a)
+    rb.run(a, 5)
+    for k, (sp, b) in enumerate(zip(specs, data)):  # each replica alone, in workgroups of 256
+        one = pdx.ReplicaBatch([sp], block=256)
+        s1 = replicas.device_state(b)
+        one.forces(s1)
+        one.run(s1, 5)
+        for t in ("x", "y", "z", "vx", "vy", "vz", "fx", "fy", "fz"):
+            for at in (k, len(rb.specs) - len(specs) + k):
+                lo, hi = int(rb.offsets[at]), int(rb.offsets[at + 1])
+                assert torch.equal(a[t][lo:hi], s1[t]), (t, at)
