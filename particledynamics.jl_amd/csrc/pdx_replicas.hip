@@ -541,10 +541,12 @@ extern "C" int pdx_replicas_destroy(pdx_rep_t r) {
 
 extern "C" int pdx_replicas_set_launch(pdx_rep_t r, int32_t block, int32_t stencil) {
   if (!r) return fail(PDX_ERR_ARGUMENT, "null handle");
-  if (block != 256 && block != 512 && block != 1024) return fail(PDX_ERR_ARGUMENT, "block must be 256, 512 or 1024");
-  if (stencil != 1 && stencil != 2) return fail(PDX_ERR_ARGUMENT, "stencil must be 1 or 2");
-  r->block = block;
-  r->block_given = true;
+  if (block != 0 && block != 256 && block != 512 && block != 1024)
+    return fail(PDX_ERR_ARGUMENT, "block must be 256, 512 or 1024 (0: by the replicas' sizes)");
+  if (stencil != 0 && stencil != 1 && stencil != 2)
+    return fail(PDX_ERR_ARGUMENT, "stencil must be 1 or 2 (0: per replica)");
+  r->block_given = block != 0;
+  r->block = block ? block : default_block(r->host);
   return stencil == r->stencil ? PDX_OK : layout(r, stencil);
 }
 

@@ -86,6 +86,7 @@ class ReplicaBatch:
         return dict(zip(keys, [int(v) for v in o]))
 
     def set_launch(self, block, stencil):
+        """Workgroup size and cells per cutoff of later runs; 0 returns to the default."""
         L.check(L.lib.pdx_replicas_set_launch(self._h, int(block), int(stencil)))
 
     def run(self, state, nsteps, dt=0.005, mass=1.0, energy=False, forces_valid=True, out=None, stream=None):
@@ -126,12 +127,12 @@ def clone_state(state):
 
 
 def autotune(batch: ReplicaBatch, state, steps=20, candidates=None, table=None, key=None, dt=0.005, mass=1.0):
-    """Pick the fastest launch shape (workgroup size, cells per cutoff) for this batch by
+    """Pick the fastest launch shape (workgroup size, cells per cutoff; 0: the default) for this batch by
     timing ``steps`` steps of each candidate on a scratch copy of ``state``; the winner is
     set on ``batch``. With ``table`` (a JSON path) results are looked up / stored under
     ``key`` (default: a signature of the batch's sizes and models). Returns (choice, timings)."""
     import torch
-    candidates = candidates or [(b, s) for s in (1, 2) for b in (256, 512, 1024)]
+    candidates = candidates or [(0, 0)] + [(b, s) for s in (0, 1, 2) for b in (256, 512, 1024)]
     if key is None:
         ns = np.array([s["n"] for s in batch.specs])
         models = "".join(sorted({s["model"][0] for s in batch.specs}))

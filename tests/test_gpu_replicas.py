@@ -305,3 +305,29 @@ def test_default_workgroup(cuda, sizes, copies, block):
             for at in (k, len(rb.specs) - len(specs) + k):
                 lo, hi = int(rb.offsets[at]), int(rb.offsets[at + 1])
                 assert torch.equal(a[t][lo:hi], s1[t]), (t, at)
+
+
+def test_default_shape_can_be_set_again(cuda):
+    """Shape 0, 0 returns a batch to the default it was created with, and the tuner times that default."""
+    import torch
+    b = _small_batch(seed=6, nrep=6, n_range=(200, 900))
+    rb = pdx.ReplicaBatch(b["specs"])
+    st = replicas.device_state(b)
+    first = rb.info()
+    rb.forces(st)
+    ref = replicas.clone_state(st)
+    rb.run(ref, 10)
+    rb.set_launch(256, 1)
+    assert (rb.info()["block"], rb.info()["stencil"]) == (256, 1)
+    rb.set_launch(first["block"], first["stencil"])
+    rb.set_launch(0, 0)
+    assert rb.info() == first
+    t = replicas.clone_state(st)
+    rb.run(t, 10)
+    for n in t:
+        assert torch.equal(t[n], ref[n]), n
+    for bad in ((128, 1), (-1, 0), (256, 3)):
+        with pytest.raises(pdx.ArgumentError):
+            rb.set_launch(*bad)
+    best, times = replicas.autotune(rb, st, steps=2)
+    assert "0x0" in times and times[f"{best[0]}x{best[1]}"] == min(times.values())
