@@ -188,8 +188,10 @@ int pdx_nl_resize_capacity(pdx_nl_t nl, int32_t cap);
 /* Change the box (set_device_box!, :89-116); the next check rebuilds. Host boundary. */
 int pdx_nl_set_box(pdx_nl_t nl, const double box[3], pdx_stream_t stream);
 /* Lanes per particle of the row build (the builder lanes of ENGINE_SETTINGS, src/engine/
- * StateEngine.jl:7-27): 1, 2, 4, 8, 16 or 32; the default fills about 2^19 threads. The rows are
- * the same set per particle whatever the lanes. A launch shape, set before capturing a graph. */
+ * StateEngine.jl:7-27): 1, 2, 4, 8, 16 or 32 lanes search each particle's stencil. 0, the default:
+ * automatic, lanes that fill about 2^19 threads, or a workgroup per cell where many cells are well
+ * filled. The rows are the same set per particle either way. A launch shape, set before capturing
+ * a graph. */
 int pdx_nl_set_row_lanes(pdx_nl_t nl, int32_t lanes);
 /* Boundary readback of the state words (device_neighbor_status, :639-651). Synchronises
  * `stream`. Returns PDX_ERR_CAPACITY / PDX_ERR_COORDINATE / PDX_ERR_STATE when check != 0
@@ -590,7 +592,7 @@ typedef struct pdx_rep_s *pdx_rep_t;
 int pdx_replicas_create(int32_t nrep, const pdx_replica_spec *specs, int32_t block, int32_t stencil,
                         pdx_rep_t *out);
 int pdx_replicas_destroy(pdx_rep_t r);
-/* Launch shape for later runs (the autotuner's knob). */
+/* Launch shape for later runs (the autotuner's knob); 0 returns to the default of pdx_replicas_create. */
 int pdx_replicas_set_launch(pdx_rep_t r, int32_t block, int32_t stencil);
 /* out: total atoms, replicas, largest replica, LDS bytes per workgroup, block, stencil as given,
  * replicas on all pairs, largest cell count. */

@@ -280,6 +280,8 @@ struct pdx_nl_s {
   int32_t interval = 20;
   int32_t row_lanes = 1;  // lanes per particle of k_rows
   bool row_lanes_given = false;  // a caller's choice: k_rows builds the rows
+  int32_t row_lanes_auto = 1;    // what lanes 0 returns to
+  bool row_lanes_env = false;
   bool allpairs = false, diagnostics = false;
   int dim = 3;  // 2: no z coordinates (z = 0), box[2] is the list's own z extent of three radii
   double box[3] = {0, 0, 0};

@@ -1243,7 +1243,8 @@ extern "C" int pdx_nl_create(int32_t n, const double box[3], double cutoff, doub
         nl->row_lanes_given = true;
       }
     }
-    nl->row_lanes = G;
+    nl->row_lanes = nl->row_lanes_auto = G;
+    nl->row_lanes_env = nl->row_lanes_given;
   }
   const int nb = blocks_for(n, TPB);
   nl->ndisp = nb;
@@ -1509,9 +1510,9 @@ extern "C" int pdx_nl_status(pdx_nl_t nl, int64_t state[PDX_DN_NSTATE], int32_t 
 
 extern "C" int pdx_nl_set_row_lanes(pdx_nl_t nl, int32_t lanes) {
   if (!nl) return fail(PDX_ERR_ARGUMENT, "null neighbor list");
-  if (lanes != 1 && lanes != 2 && lanes != 4 && lanes != 8 && lanes != 16 && lanes != 32)
-    return fail(PDX_ERR_ARGUMENT, "row-build lanes must be 1, 2, 4, 8, 16 or 32");
-  nl->row_lanes = lanes;
-  nl->row_lanes_given = true;
+  if (lanes != 0 && lanes != 1 && lanes != 2 && lanes != 4 && lanes != 8 && lanes != 16 && lanes != 32)
+    return fail(PDX_ERR_ARGUMENT, "row-build lanes must be 1, 2, 4, 8, 16 or 32 (0: automatic)");
+  nl->row_lanes = lanes ? lanes : nl->row_lanes_auto;
+  nl->row_lanes_given = lanes ? true : nl->row_lanes_env;
   return PDX_OK;
 }

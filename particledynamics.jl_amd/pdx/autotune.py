@@ -4,7 +4,7 @@ neighbours-per-atom class, the measured best builder lanes, force lanes, skin an
 
 Here a setting holds the knobs of one ``ForceEngine`` evaluation:
   * ``force_lanes``: lanes per particle of the pair kernel's row traversal;
-  * ``build_lanes``: lanes per particle of the row build;
+  * ``build_lanes``: lanes per particle of the row build (0: automatic);
   * ``overlap``: how the pair kernel shares the device with the mesh branch ("fft": it waits for
     the spread and runs beside the transforms; "spread": it runs beside the whole mesh branch);
   * ``spread_threads``, ``transform_threads``: workgroup sizes of the owner-computes spread that
@@ -81,7 +81,7 @@ def apply(engine, setting):
         raise L.ArgumentError("settings apply to the ELL backend")
     if "force_lanes" in setting:
         engine.pairs.set_lanes(int(setting["force_lanes"]))
-    if setting.get("build_lanes"):
+    if "build_lanes" in setting:
         engine.nl.set_row_lanes(int(setting["build_lanes"]))
     if "overlap" in setting:
         if setting["overlap"] not in ("spread", "solve", "fft"):

@@ -105,7 +105,8 @@ class DeviceNeighborWorkspace:
         return perm.long()
 
     def set_row_lanes(self, lanes: int):
-        """Lanes per particle of the row build (the builder lanes of the engine settings)."""
+        """Lanes per particle of the row build (the builder lanes of the engine settings); 0 returns to
+        the automatic build."""
         L.check(L.lib.pdx_nl_set_row_lanes(self._h, int(lanes)))
         self.row_lanes_set = int(lanes)
 

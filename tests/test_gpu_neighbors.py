@@ -315,3 +315,31 @@ def test_cell_order_at_the_launch_rules(cuda, grid, N):
     fits = int(ws.counts().max()) <= ws.cap
     assert (s[6], s[9], s[10]) == (3, 2, 2) and (s[1], s[7]) == ((1, 2) if fits else (0, 1))
     check()
+
+
+def test_row_lanes_return_to_automatic(cuda):
+    """Lanes 0 is the automatic build again, through the list and through a tuner's setting; the rows are
+    the same."""
+    import torch
+    from pdx import autotune
+    box, N = (31.0, 31.0, 31.0), 16000
+    rng = np.random.default_rng(1)
+    X, Y, Z = (dev(((rng.random(N) - 0.5) * 31.0).astype(np.float32)) for _ in range(3))
+    eng = pdx.ForceEngine(N, box, pdx.LennardJones(epsilon=1e-6), skin=0.5)
+    f = [torch.empty(N, device="cuda") for _ in range(3)]
+    rows = []
+    for lanes in (None, 8, 0):
+        if lanes is not None:
+            autotune.apply(eng, {"build_lanes": lanes})
+            assert autotune.current(eng)["build_lanes"] == lanes
+        eng.nl.invalidate()
+        eng.evaluate(X, Y, Z, None, *f, None, None, energy=False)
+        eng.nl.status()
+        cnt = eng.nl.counts()
+        keep = torch.arange(eng.nl.cap, device="cuda")[:, None] < cnt[None, :]
+        rows.append((cnt.clone(), torch.where(keep, eng.nl.neighbors_flat(), torch.zeros_like(eng.nl.neighbors_flat()))))
+    for c, r in rows[1:]:
+        assert torch.equal(c, rows[0][0]) and torch.equal(r, rows[0][1])
+    for bad in (-1, 3, 64):
+        with pytest.raises(pdx.ArgumentError):
+            eng.nl.set_row_lanes(bad)
