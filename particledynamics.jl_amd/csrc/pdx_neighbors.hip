@@ -20,6 +20,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
+#include <mutex>
 
 using namespace pdx;
 
@@ -241,7 +242,7 @@ __global__ __launch_bounds__(TPB) void k_bin(int N, const float4 *__restrict__ p
 // run totals; the counts come from the caches) and places its share of the particles; workgroup 0
 // stores the offsets and, with DECIDE, writes k_bin's decision into the state words, which the other
 // workgroups do not read.
-constexpr int SCAN_FUSED_MAX = 16000;  // 62.5 KiB of LDS
+constexpr int SCAN_FUSED_MAX = 16384;  // 64 KiB of LDS
 constexpr int SCAN_THREADS = 1024;
 constexpr int SCAN_GRID = 64;  // 16 and 256 are 1% slower (256 000 LJ atoms), 1 is 10%
 template <bool DECIDE>
@@ -290,6 +291,19 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_scan_scatter(int ncell, int N,
   }
   for (int i = blockIdx.x * SCAN_THREADS + threadIdx.x; i < N; i += gridDim.x * SCAN_THREADS)
     ids_sorted[first[cell_of_particle[i]] - 1 + cell_rank[i]] = i + 1;
+}
+
+// The largest grids pass the 64 KiB a launch may take unasked.
+void allow_scan_lds() {
+  static std::once_flag once;
+  std::call_once(once, [] {
+    const int most = sizeof(int32_t) * SCAN_FUSED_MAX;
+    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_scan_scatter<false>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, most);
+    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_scan_scatter<true>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, most);
+    (void)hipGetLastError();
+  });
 }
 
 // Exclusive scan of cell_counts, SCAN_BLOCK cells per block (block-local part).
@@ -1246,6 +1260,7 @@ extern "C" int pdx_nl_create(int32_t n, const double box[3], double cutoff, doub
     nl->row_lanes = nl->row_lanes_auto = G;
     nl->row_lanes_env = nl->row_lanes_given;
   }
+  allow_scan_lds();
   const int nb = blocks_for(n, TPB);
   nl->ndisp = nb;
   const int cb = std::max(blocks_for((int64_t)n * 32, TPB), 8192);  // the row kernels' largest grids

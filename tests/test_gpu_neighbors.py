@@ -270,11 +270,12 @@ def test_rows_of_dense_cells_equal_row_search(cuda, grid, clump):
 
 
 @pytest.mark.parametrize("grid,N", [((3, 3, 3), 1), ((4, 5, 6), 1025), ((24, 24, 24), 262144), ((24, 24, 24), 262145),
-                                    ((20, 20, 40), 65537), ((20, 20, 41), 65537)])
+                                    ((20, 20, 40), 65537), ((20, 20, 41), 65537), ((16, 32, 32), 65537),
+                                    ((5, 29, 113), 65537)])
 def test_cell_order_at_the_launch_rules(cuda, grid, N):
     """Cells, offsets and sorted ids of a build, and the decision to build, on both sides of the sizes
     where the binning takes the decision (262 144 particles) and the scan shares the scatter's launch
-    (16 000 cells)."""
+    (16 384 cells)."""
     import torch
     w = 3.001
     box = tuple(w * g for g in grid)
