@@ -459,7 +459,8 @@ __device__ __forceinline__ void row_partials(int longest, long long tested, long
   __syncthreads();
   if (threadIdx.x == 0) {
     for (int k = 1; k < nw; ++k) { longest = max(longest, smax[k]); tested += ssum[0][k]; accepted += ssum[1][k]; }
-    atomicMax(row_max, longest);
+    // most blocks find a longer row already there: their atomics would only queue for the one word
+    if (longest > __hip_atomic_load(row_max, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(row_max, longest);
     stat_partial[2 * blockIdx.x] = tested;
     stat_partial[2 * blockIdx.x + 1] = accepted;
   }
