@@ -298,7 +298,7 @@ struct pdx_nl_s {
   pdx::DevBuf<float> disp_partial;  // ndisp per-block maxima of the last check
   int32_t ndisp = 0;
   pdx::DevBuf<int64_t> decision;      // the check's decision on its way to the state words
-  pdx::DevBuf<int32_t> row_max;       // largest row of the build under way
+  pdx::DevBuf<int32_t> row_max;       // of the build under way: largest rows, masks_pay's choice
   pdx::DevBuf<int64_t> stat_partial;  // 2 per row block: candidates, accepted
   pdx::DevBuf<int32_t> scan_block;    // per-1024-cell block totals
   pdx::DevBuf<int64_t> candidates;    // N (diagnostics)
@@ -311,6 +311,7 @@ struct pdx_nl_s {
   int snap_host = 0;  // checks since create / box change (capped at 2): at 2 a snapshot was taken
   const void *packed_src[4] = {nullptr, nullptr, nullptr, nullptr};  // x, y, z, q of the last check
   int check_force = 0;  // the last check was a forced rebuild (pdx_nl_rebuild)
+  pdx::DevBuf<int2> scan_occ;  // per-1024-cell blocks' occupied cells and largest cell
 };
 
 struct pdx_pair_s {

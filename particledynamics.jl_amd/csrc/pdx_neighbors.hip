@@ -12,7 +12,7 @@
 //                  (k_scan_local / k_scan_blocks / k_scan_finish / k_scatter above SCAN_FUSED_MAX cells)
 //   k_sort_cells   ascending id inside each cell (rows and traversal become reproducible),
 //                  and the cell-ordered packed positions read by the row kernel
-//   k_rows_masks   (or k_rows / k_rows_cells / k_rows_allpairs) 27-cell stencil, r^2 <= rlist^2,
+//   k_rows_auto    (or k_rows / k_rows_cells / k_rows_allpairs) 27-cell stencil, r^2 <= rlist^2,
 //                  slot-major rows t*N + i, 1-based ids; per-block max row length and statistics
 //   k_commit_refs  max row length vs cap, state words; reference positions of a successful build
 #include "pdx_internal.hpp"
@@ -27,6 +27,12 @@ using namespace pdx;
 namespace {
 
 constexpr int TPB = 256;
+// The longest row is kept in ROW_WORDS words, one a cache line: one word is a queue of atomics from all
+// row workgroups (rebuilds of 10 240 particles on 8^3 cells 58 us, with them 52), and a workgroup that
+// looked first would wait for it (rows of 256 000 LJ atoms 204 us against 200).
+constexpr int ROW_WORDS = 64;
+constexpr int ROW_LINE = 32;                       // words of a cache line
+constexpr int ROW_CHOICE = ROW_WORDS * ROW_LINE;  // word of masks_pay's choice
 constexpr int DECIDE_BLOCKS = 1024;  // check blocks of a list whose k_bin decides
 constexpr int SCAN_BLOCK = 1024;  // cells per block of the local scan (256 threads x 4)
 
@@ -108,7 +114,7 @@ __global__ __launch_bounds__(TPB) void k_decide(int N, float *__restrict__ x,
     packed[i] = make_float4(c[0], c[1], c[2], q ? q[i] : 0.0f);
   }
   // histogram and largest row are scratch of the next rebuild: cleared here (one launch fewer)
-  if (i == 0) *row_max = 0;
+  if (i < ROW_WORDS) row_max[i * ROW_LINE] = 0;
   if (!allpairs)
     for (int c = i; c < ncell; c += gridDim.x * TPB) cell_counts[c] = 0;
 
@@ -236,6 +242,28 @@ __global__ __launch_bounds__(TPB) void k_bin(int N, const float4 *__restrict__ p
   cell_rank[i] = atomicAdd(&cell_counts[c], 1);
 }
 
+// Where mask_rows is the faster build, by how the particles fill the cells now (occupied cells, largest
+// cell): a workgroup per cell needs cells enough for the CUs, and no cell far above the mean one, on which
+// the launch would wait. Whole rebuilds in microseconds, masks against k_rows at its default lanes:
+// random particles in cell order, 1 331 cells of 14, 30, 60, 72, 80: 56 / 91 / 284 / 428 / 504 against
+// 76 / 109 / 337 / 427 / 407; 8 000 cells of 14, 60, 100, 120: 133 / 1 169 / 3 545 / 5 323 against
+// 137 / 1 307 / 3 682 / 5 267; a droplet of 61 440 particles in 1 000 of 4 096 cells 256 against 197, in
+// 2 742 of them 103 against 121; half of 43 904 in a blob of 350 a cell 1 888 against 426. Two-dimensional
+// lists have a third of the stencil: 1 600 occupied cells of 43 and 60: 140 / 243 against 137 / 211;
+// 2 500: 162 / 298 against 172 / 384.
+__device__ __forceinline__ bool masks_pay(int N, int ncell, bool flat, int used, int largest) {
+  const long long n = N;
+  if (used < (flat ? 2048 : 1024) || (long long)largest * used > 2 * n + 16ll * used) return false;
+  return n <= (long long)used * (used >= 4096 || flat ? 100 : (used == ncell ? 72 : 56));
+}
+
+// Occupied cells and the largest one of a wave's lanes.
+__device__ __forceinline__ int2 occupancy(int used, int largest) {
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) used += __shfl_xor(used, off, WAVE);
+  return make_int2(used, wave_max(largest));
+}
+
 // Cell offsets (1-based, last entry N+1: _device_offsets_kernel!, DeviceNeighborCUDA.jl:280-289) and
 // the particles' scatter in one launch for grids of up to SCAN_FUSED_MAX cells: every workgroup scans
 // all counts in its LDS (1024 threads, a contiguous run of at most 16 cells each, wave scans of the
@@ -250,7 +278,8 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_scan_scatter(int ncell, int N,
                                                                int32_t *offsets,
                                                                const int32_t *__restrict__ cell_of_particle,
                                                                const int32_t *__restrict__ cell_rank,
-                                                               int32_t *ids_sorted, int64_t *state,
+                                                               int32_t *ids_sorted, int32_t *row_max, int flat,
+                                                               int64_t *state,
                                                                const Decision *__restrict__ decision) {
   if (DECIDE) {
     const Decision d = *decision;
@@ -262,13 +291,25 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_scan_scatter(int ncell, int N,
   }
   extern __shared__ int32_t first[];  // ncell
   __shared__ int32_t wtot[SCAN_THREADS / WAVE];
+  __shared__ int2 wocc[SCAN_THREADS / WAVE];
+  int used = 0, largest = 0;
   for (int c = threadIdx.x; c < ncell; c += SCAN_THREADS) first[c] = counts[c];
   __syncthreads();
   const int per = (ncell + SCAN_THREADS - 1) / SCAN_THREADS;
   const int c0 = min((int)threadIdx.x * per, ncell), c1 = min(c0 + per, ncell);
   int32_t run = 0;
-  for (int c = c0; c < c1; ++c) run += first[c];
+  for (int c = c0; c < c1; ++c) {
+    const int n = first[c];
+    run += n;
+    used += n != 0;
+    largest = max(largest, n);
+  }
   const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
+  const bool choose = blockIdx.x == gridDim.x - 1;  // (workgroup 0 stores the offsets)
+  if (choose) {
+    const int2 o = occupancy(used, largest);
+    if (lane == 0) wocc[w] = o;
+  }
   int32_t v = run;
 #pragma unroll
   for (int o = 1; o < WAVE; o <<= 1) {
@@ -288,6 +329,10 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_scan_scatter(int ncell, int N,
   if (blockIdx.x == 0) {
     for (int c = threadIdx.x; c < ncell; c += SCAN_THREADS) offsets[c] = first[c];
     if (threadIdx.x == 0) offsets[ncell] = N + 1;
+  }
+  if (choose && w == 0) {
+    const int2 o = lane < SCAN_THREADS / WAVE ? wocc[lane] : make_int2(0, 0), all = occupancy(o.x, o.y);
+    if (lane == 0) row_max[ROW_CHOICE] = masks_pay(N, ncell, flat != 0, all.x, all.y);
   }
   for (int i = blockIdx.x * SCAN_THREADS + threadIdx.x; i < N; i += gridDim.x * SCAN_THREADS)
     ids_sorted[first[cell_of_particle[i]] - 1 + cell_rank[i]] = i + 1;
@@ -309,9 +354,11 @@ void allow_scan_lds() {
 // Exclusive scan of cell_counts, SCAN_BLOCK cells per block (block-local part).
 __global__ __launch_bounds__(TPB) void k_scan_local(int ncell, const int32_t *counts,
                                                      int32_t *offsets, int32_t *block_totals,
-                                                     const int64_t *state) {
+                                                     int2 *block_occ, const int64_t *state) {
   if (!rebuild_requested(state)) return;
   __shared__ int32_t sh[TPB];
+  __shared__ int2 wocc[TPB / WAVE];
+  int used = 0, largest = 0;
   const int base = blockIdx.x * SCAN_BLOCK + threadIdx.x * 4;
   int32_t v[4];
   int32_t run = 0;
@@ -319,7 +366,11 @@ __global__ __launch_bounds__(TPB) void k_scan_local(int ncell, const int32_t *co
   for (int k = 0; k < 4; ++k) {
     v[k] = (base + k < ncell) ? counts[base + k] : 0;
     run += v[k];
+    used += v[k] != 0;
+    largest = max(largest, v[k]);
   }
+  const int2 o = occupancy(used, largest);
+  if ((threadIdx.x & (WAVE - 1)) == 0) wocc[threadIdx.x / WAVE] = o;
   sh[threadIdx.x] = run;
   __syncthreads();
   for (int off = 1; off < TPB; off <<= 1) {
@@ -334,14 +385,34 @@ __global__ __launch_bounds__(TPB) void k_scan_local(int ncell, const int32_t *co
     if (base + k < ncell) offsets[base + k] = excl;
     excl += v[k];
   }
-  if (threadIdx.x == TPB - 1) block_totals[blockIdx.x] = sh[TPB - 1];
+  if (threadIdx.x == TPB - 1) {
+    block_totals[blockIdx.x] = sh[TPB - 1];
+    int2 t = wocc[0];
+    for (int k = 1; k < TPB / WAVE; ++k) t = make_int2(t.x + wocc[k].x, max(t.y, wocc[k].y));
+    block_occ[blockIdx.x] = t;
+  }
 }
 
-// Exclusive scan of the block totals (one block, sequential over chunks of 1024).
+// Exclusive scan of the block totals (one block, sequential over chunks of 1024), and the grid's occupancy.
 __global__ __launch_bounds__(1024) void k_scan_blocks(int nblocks, int32_t *block_totals,
+                                                       const int2 *__restrict__ block_occ, int32_t *row_max,
+                                                       int N, int ncell, int flat,
                                                        const int64_t *state) {
   if (!rebuild_requested(state)) return;
   __shared__ int32_t sh[1024];
+  __shared__ int2 wocc[1024 / WAVE];
+  int used = 0, largest = 0;
+  for (int k = threadIdx.x; k < nblocks; k += 1024) {
+    used += block_occ[k].x;
+    largest = max(largest, block_occ[k].y);
+  }
+  const int2 o = occupancy(used, largest);
+  if ((threadIdx.x & (WAVE - 1)) == 0) wocc[threadIdx.x / WAVE] = o;
+  __syncthreads();
+  if (threadIdx.x < WAVE) {
+    const int2 t = threadIdx.x < 1024 / WAVE ? wocc[threadIdx.x] : make_int2(0, 0), all = occupancy(t.x, t.y);
+    if (threadIdx.x == 0) row_max[ROW_CHOICE] = masks_pay(N, ncell, flat != 0, all.x, all.y);
+  }
   int32_t carry = 0;
   for (int base = 0; base < nblocks; base += 1024) {
     const int k = base + threadIdx.x;
@@ -430,21 +501,8 @@ __global__ __launch_bounds__(WAVE) void k_sort_cells(int ncell, const int32_t *o
 }
 
 // ------------------------------------------------------------------ rows
-// G lanes per particle, particles in cell order (the groups of a wave share their home cell,
-// so candidate loads are broadcast). The group walks the 27-cell stencil G candidates at a
-// time; accepted neighbours are placed with a wave64 ballot + popcount in candidate order, so
-// every row is identical whatever G is. Distance test as the reference: mic_fast differences,
-// r^2 = muladd(dx,dx,muladd(dy,dy,dz^2)) <= rl^2 (_kernel_neighbors3!, DenseNeighborCUDA.jl:153-206;
-// cooperative placement as _cooperative_rows3_kernel!, src/engine/Builder.jl:39-129). Slots are
-// written slot-major at t*N + i with 1-based ids; the count keeps growing past cap so the
-// commit can report the required capacity.
-// STAGE (opt-in): the workgroup's rows are kept in LDS as [slot][particle] (TPB/G particles, cap
-// slots, at most 64 KiB) and written out slot by slot after the search, so a row slot of
-// consecutive particles is one contiguous store; written straight from the search, the slots of
-// a wave's particles advance at different rates and the 4-byte stores land in partially filled
-// lines (measured: 8.6x the row bytes at 486 400 ions, 2.0x staged). Same rows either way.
 // Commit data of a block's rows (_device_capacity_partial_kernel!, DeviceNeighborCUDA.jl:291-310): the
-// largest row into one word, candidates and accepted entries per block; called by every thread.
+// largest row into a word of its group, candidates and accepted entries per block; called by every thread.
 __device__ __forceinline__ void row_partials(int longest, long long tested, long long accepted, int32_t *row_max,
                                              int64_t *stat_partial) {
   __shared__ int smax[TPB / WAVE];
@@ -459,30 +517,37 @@ __device__ __forceinline__ void row_partials(int longest, long long tested, long
   __syncthreads();
   if (threadIdx.x == 0) {
     for (int k = 1; k < nw; ++k) { longest = max(longest, smax[k]); tested += ssum[0][k]; accepted += ssum[1][k]; }
-    // most blocks find a longer row already there: their atomics would only queue for the one word
-    if (longest > __hip_atomic_load(row_max, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(row_max, longest);
+    atomicMax(&row_max[(blockIdx.x % ROW_WORDS) * ROW_LINE], longest);
     stat_partial[2 * blockIdx.x] = tested;
     stat_partial[2 * blockIdx.x + 1] = accepted;
   }
 }
 
+// G lanes per particle, particles in cell order (the groups of a wave share their home cell,
+// so candidate loads are broadcast). The group walks the 27-cell stencil G candidates at a
+// time; accepted neighbours are placed with a wave64 ballot + popcount in candidate order, so
+// every row is identical whatever G is. Distance test as the reference: mic_fast differences,
+// r^2 = muladd(dx,dx,muladd(dy,dy,dz^2)) <= rl^2 (_kernel_neighbors3!, DenseNeighborCUDA.jl:153-206;
+// cooperative placement as _cooperative_rows3_kernel!, src/engine/Builder.jl:39-129). Slots are
+// written slot-major at t*N + i with 1-based ids; the count keeps growing past cap so the
+// commit can report the required capacity.
+// STAGE (opt-in): the workgroup's rows are kept in LDS as [slot][particle] (TPB/G particles, cap
+// slots, at most 64 KiB) and written out slot by slot after the search, so a row slot of
+// consecutive particles is one contiguous store; written straight from the search, the slots of
+// a wave's particles advance at different rates and the 4-byte stores land in partially filled
+// lines (measured: 8.6x the row bytes at 486 400 ions, 2.0x staged). Same rows either way.
 constexpr size_t ROW_STAGE_BYTES = 65536;
+// The rows of the vb-th TPB / G particles; longest, all_tested and all_found take this thread's rows.
 template <int G, bool STAGE>
-__global__ __launch_bounds__(TPB) void k_rows(int N, int cap, int nx, int ny, int nz,
-                                               const float4 *__restrict__ sorted,
-                                               const int32_t *__restrict__ offsets,
-                                               const int32_t *__restrict__ cell_of_particle,
-                                               const float *geom, float rl2, int32_t *nbr,
-                                               int32_t *counts, int64_t *candidates, int32_t *row_max,
-                                               int64_t *stat_partial, const int64_t *state) {
+__device__ __forceinline__ void search_rows(int vb, int N, int cap, int nx, int ny, int nz,
+                                            const float4 *__restrict__ sorted, const int32_t *__restrict__ offsets,
+                                            const int32_t *__restrict__ cell_of_particle, const float *geom, float rl2,
+                                            int32_t *nbr, int32_t *counts, int64_t *candidates, int &longest,
+                                            long long &all_tested, long long &all_found) {
   constexpr int PB = TPB / G;  // particles per workgroup
   extern __shared__ int32_t srow[];  // STAGE: [cap][PB]
-  __shared__ int sfound[PB], sid[PB];
-  __shared__ int smax;
-  if (!rebuild_requested(state)) return;  // uniform over the grid
-  const int gid = blockIdx.x * TPB + threadIdx.x;
-  const int t = gid / G;
-  const int lg = gid % G;
+  const int t = vb * PB + threadIdx.x / G;
+  const int lg = threadIdx.x % G;
   const int pb = threadIdx.x / G;
   const int wl = threadIdx.x & (WAVE - 1);
   const unsigned long long gmask = (G == WAVE) ? ~0ull : (((1ull << G) - 1ull) << (wl - lg));
@@ -546,6 +611,8 @@ __global__ __launch_bounds__(TPB) void k_rows(int N, int cap, int nx, int ny, in
     }
   }
   if (STAGE) {
+    __shared__ int sfound[PB], sid[PB];
+    __shared__ int smax;
     if (lg == 0) {
       sfound[pb] = active ? min(found, cap) : 0;
       sid[pb] = i;
@@ -563,9 +630,26 @@ __global__ __launch_bounds__(TPB) void k_rows(int N, int cap, int nx, int ny, in
   if (active && lg == 0) {
     counts[i] = found;
     if (candidates) candidates[i] = tested;
+    longest = max(longest, found);
+    all_tested += tested;
+    all_found += found;
   }
-  const bool own = active && lg == 0;
-  row_partials(own ? found : 0, own ? tested : 0, own ? found : 0, row_max, stat_partial);
+}
+
+template <int G, bool STAGE>
+__global__ __launch_bounds__(TPB) void k_rows(int N, int cap, int nx, int ny, int nz,
+                                               const float4 *__restrict__ sorted,
+                                               const int32_t *__restrict__ offsets,
+                                               const int32_t *__restrict__ cell_of_particle,
+                                               const float *geom, float rl2, int32_t *nbr,
+                                               int32_t *counts, int64_t *candidates, int32_t *row_max,
+                                               int64_t *stat_partial, const int64_t *state) {
+  if (!rebuild_requested(state)) return;  // uniform over the grid
+  int longest = 0;
+  long long all_tested = 0, all_found = 0;
+  search_rows<G, STAGE>(blockIdx.x, N, cap, nx, ny, nz, sorted, offsets, cell_of_particle, geom, rl2, nbr, counts,
+                        candidates, longest, all_tested, all_found);
+  row_partials(longest, all_tested, all_found, row_max, stat_partial);
 }
 
 // Rows from LDS-staged candidates: one workgroup per cell. Wave 0 lists the cell's 27 stencil cells
@@ -687,7 +771,7 @@ __global__ __launch_bounds__(TPB) void k_rows_cells(int N, int cap, int ncell, i
   row_partials(longest, all_tested, all_found, row_max, stat_partial);
 }
 
-// ---- the default build of many well-filled cells: one workgroup per cell, lanes = candidates,
+// ---- the build of many evenly filled cells: one workgroup per cell, lanes = candidates,
 // particles one after the other in scalar registers (four waves, a chunk of 64 candidates each in
 // turn). A distance test of 64 candidates is then seven vector instructions (three more per
 // dimension where the stencil crosses the seam), its ballot goes into lane p of a register pair (particle p of the cell), and the cell's tests end as bit
@@ -705,23 +789,18 @@ __global__ __launch_bounds__(TPB) void k_rows_cells(int N, int cap, int ncell, i
 extern "C" __device__ __attribute__((const)) int pdx_writelane(int value, int lane, int old) __asm("llvm.amdgcn.writelane.i32");
 constexpr int RM_CHUNKS = 28;  // candidate chunks of 64 per pass (21 KiB of LDS: seven workgroups per CU)
 constexpr int RM_WAVES = TPB / WAVE;
-__global__ __launch_bounds__(TPB) void k_rows_masks(int N, int cap, int ncell, int nx, int ny, int nz,
-                                                     const float4 *__restrict__ sorted,
-                                                     const int32_t *__restrict__ offsets,
-                                                     const float *__restrict__ geom, float rl2,
-                                                     int32_t *__restrict__ nbr, int32_t *__restrict__ counts,
-                                                     int64_t *candidates, int32_t *row_max, int64_t *stat_partial,
-                                                     const int64_t *state) {
+__device__ __forceinline__ void mask_rows(int N, int cap, int ncell, int nx, int ny, int nz,
+                                          const float4 *__restrict__ sorted, const int32_t *__restrict__ offsets,
+                                          const float *__restrict__ geom, float rl2, int32_t *__restrict__ nbr,
+                                          int32_t *__restrict__ counts, int64_t *candidates, int &longest,
+                                          long long &all_tested, long long &all_found) {
   __shared__ uint2 mask[RM_CHUNKS][WAVE];
   __shared__ int32_t cid[RM_CHUNKS * WAVE];
   __shared__ int cstart[27], cpre[28], ends[WAVE];
-  if (!rebuild_requested(state)) return;  // uniform over the grid
   const int lane = threadIdx.x & (WAVE - 1);
   const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x / WAVE);
   const float Lx = geom[0], Ly = geom[1], Lz = geom[2];
   const float hx = 0.5f * Lx, hy = 0.5f * Ly, hz = 0.5f * Lz;
-  int longest = 0;
-  long long all_tested = 0, all_found = 0;
   for (int c = blockIdx.x; c < ncell; c += gridDim.x) {
     const int p0 = offsets[c] - 1, np = offsets[c + 1] - 1 - p0;  // uniform
     if (np <= 0) continue;
@@ -844,6 +923,29 @@ __global__ __launch_bounds__(TPB) void k_rows_masks(int N, int cap, int ncell, i
       }
     }
   }
+}
+
+template <int G>  // seven waves a SIMD: what the masks' LDS allows
+__global__ __launch_bounds__(TPB, 7) void k_rows_auto(int N, int cap, int ncell, int nx, int ny, int nz,
+                                                   const float4 *__restrict__ sorted,
+                                                   const int32_t *__restrict__ offsets,
+                                                   const int32_t *__restrict__ cell_of_particle,
+                                                   const float *__restrict__ geom, float rl2,
+                                                   int32_t *__restrict__ nbr, int32_t *__restrict__ counts,
+                                                   int64_t *candidates, int32_t *row_max, int64_t *stat_partial,
+                                                   const int64_t *state) {
+  const bool masks = row_max[ROW_CHOICE] != 0;  // (read beside the request)
+  if (!rebuild_requested(state)) return;  // uniform over the grid
+  int longest = 0;
+  long long all_tested = 0, all_found = 0;
+  if (__builtin_expect(masks, 1)) {
+    mask_rows(N, cap, ncell, nx, ny, nz, sorted, offsets, geom, rl2, nbr, counts, candidates, longest, all_tested,
+              all_found);
+  } else {
+    for (int vb = blockIdx.x; (long long)vb * (TPB / G) < N; vb += gridDim.x)
+      search_rows<G, false>(vb, N, cap, nx, ny, nz, sorted, offsets, cell_of_particle, geom, rl2, nbr, counts,
+                            candidates, longest, all_tested, all_found);
+  }
   row_partials(longest, all_tested, all_found, row_max, stat_partial);
 }
 
@@ -889,7 +991,8 @@ __global__ __launch_bounds__(TPB) void k_commit_refs(int N, int nblocks, int cap
                                                      const int64_t *__restrict__ stat_partial,
                                                      const float4 *__restrict__ packed, float *rref, int64_t *state) {
   if (!rebuild_requested(state)) return;
-  const int largest = *row_max;
+  static_assert(ROW_WORDS == WAVE, "one word a lane");
+  const int largest = wave_max(row_max[(threadIdx.x & (WAVE - 1)) * ROW_LINE]);
   const int i = blockIdx.x * TPB + threadIdx.x;
   if (largest <= cap && i < N) {
     const float4 p = packed[i];
@@ -1056,6 +1159,7 @@ int enqueue_decide_build(pdx_nl_t nl, hipStream_t st) {
                        nl->check_force, nl->snap_state.p, (int)nl->allpairs);
   if (!nl->allpairs) {
     const int sblocks = blocks_for(nl->ncell, SCAN_BLOCK);
+    const int flat = nl->dim == 2;
     auto bin = decide_fused ? k_bin<true> : k_bin<false>;
     hipLaunchKernelGGL(bin, dim3(nb), dim3(TPB), 0, st, N, nl->packed.p, geom, nl->nx, nl->ny, nl->nz,
                        nl->cell_of_particle.p, nl->cell_counts.p, nl->cell_rank.p, s, nb, nl->disp_partial.p,
@@ -1064,11 +1168,13 @@ int enqueue_decide_build(pdx_nl_t nl, hipStream_t st) {
       auto scan = decide_fused ? k_scan_scatter<true> : k_scan_scatter<false>;
       hipLaunchKernelGGL(scan, dim3(std::min(blocks_for(N, SCAN_THREADS), SCAN_GRID)), dim3(SCAN_THREADS),
                          sizeof(int32_t) * (size_t)nl->ncell, st, nl->ncell, N, nl->cell_counts.p, nl->cell_offsets.p,
-                         nl->cell_of_particle.p, nl->cell_rank.p, nl->particle_ids_sorted.p, s, dec);
+                         nl->cell_of_particle.p, nl->cell_rank.p, nl->particle_ids_sorted.p, nl->row_max.p, flat,
+                         s, dec);
     } else {
       hipLaunchKernelGGL(k_scan_local, dim3(sblocks), dim3(TPB), 0, st, nl->ncell, nl->cell_counts.p,
-                         nl->cell_offsets.p, nl->scan_block.p, s);
-      hipLaunchKernelGGL(k_scan_blocks, dim3(1), dim3(1024), 0, st, sblocks, nl->scan_block.p, s);
+                         nl->cell_offsets.p, nl->scan_block.p, nl->scan_occ.p, s);
+      hipLaunchKernelGGL(k_scan_blocks, dim3(1), dim3(1024), 0, st, sblocks, nl->scan_block.p,
+                         nl->scan_occ.p, nl->row_max.p, N, nl->ncell, flat, s);
       hipLaunchKernelGGL(k_scan_finish, dim3(blocks_for(nl->ncell + 1, TPB)), dim3(TPB), 0, st, nl->ncell, N,
                          nl->cell_offsets.p, nl->scan_block.p, s);
       hipLaunchKernelGGL(k_scatter, dim3(nb), dim3(TPB), 0, st, N, nl->cell_of_particle.p, nl->cell_rank.p,
@@ -1076,12 +1182,8 @@ int enqueue_decide_build(pdx_nl_t nl, hipStream_t st) {
     }
     hipLaunchKernelGGL(k_sort_cells, dim3(std::min(nl->ncell, 8192)), dim3(WAVE), 0, st, nl->ncell, nl->cell_offsets.p,
                        nl->particle_ids_sorted.p, nl->packed.p, nl->sorted.p, s);
-    // The mask build, a workgroup per cell, where there are four cells a CU and cells of 14 particles
-    // and more on average. Whole rebuilds in microseconds, masks against k_rows at its default lanes
-    // (random particles in cell order): 4 096 cells of 2, 8, 14, 60 particles 80 / 90 / 103 / 628
-    // against 53 / 73 / 109 / 726; 21 952 cells of 4, 8, 14, 30: 140 / 176 / 282 / 665 against
-    // 102 / 152 / 330 / 988; 1 000 cells of 60: 230 against 208. k_rows also takes a caller's lane
-    // count and the opt-in forms below.
+    // Lists of 14 to 100 particles a cell on at least 1 024 cells choose between the mask build and
+    // k_rows on the device (masks_pay); k_rows also takes a caller's lane count and the opt-in forms below.
     // Lanes per particle of k_rows: the list's row lanes; with PDX_ROW_STAGE=1 the rows are staged in LDS and
     // the lanes raised until the workgroup's rows fit the 64 KiB stage. Staging cuts the build's HBM
     // writes at 486 400 ions from 3.97 GB to 0.93 GB but not its time (1.13 ms at 32 lanes against
@@ -1091,16 +1193,27 @@ int enqueue_decide_build(pdx_nl_t nl, hipStream_t st) {
     if (const char *v = std::getenv("PDX_ROW_STAGE")) stage = std::atoi(v) != 0;
     // the cell-staged build (k_rows_cells, PDX_ROW_CELLS=1): at 486 400 ions (8 000 cells, one
     // workgroup each) 1.06-1.09 ms against 1.12 ms for k_rows in spatial storage order, 1.33 against
-    // 1.55 ms in lattice order; a whole rebuild with k_rows_masks takes 1.02 ms, with k_rows 1.22
+    // 1.55 ms in lattice order; a whole rebuild with mask_rows takes 1.02 ms, with k_rows 1.22
     bool cells = false;
     if (const char *v = std::getenv("PDX_ROW_CELLS")) cells = std::atoi(v) != 0;
     if (stage) cells = false;
-    const bool masks = !stage && !cells && !nl->row_lanes_given && nl->ncell >= 1024 && N >= 14 * (int64_t)nl->ncell;
-    if (masks) {
+    if (!stage && !cells && !nl->row_lanes_given && nl->ncell >= 1024 && N >= 14 * (int64_t)nl->ncell &&
+        N <= 100 * (int64_t)nl->ncell) {
       row_blocks = std::min(nl->ncell, 4096);
-      hipLaunchKernelGGL(k_rows_masks, dim3(row_blocks), dim3(TPB), 0, st, N, nl->cap, nl->ncell, nl->nx, nl->ny,
-                         nl->nz, nl->sorted.p, nl->cell_offsets.p, geom, nl->rl2, nl->neighbors_flat.p, nl->counts.p,
-                         nl->diagnostics ? nl->candidates.p : nullptr, nl->row_max.p, nl->stat_partial.p, s);
+#define PDX_ROWA(GG)                                                                                            \
+  hipLaunchKernelGGL((k_rows_auto<GG>), dim3(row_blocks), dim3(TPB), 0, st, N, nl->cap, nl->ncell, nl->nx,      \
+                     nl->ny, nl->nz, nl->sorted.p, nl->cell_offsets.p, nl->cell_of_particle.p, geom, nl->rl2,   \
+                     nl->neighbors_flat.p, nl->counts.p, nl->diagnostics ? nl->candidates.p : nullptr,          \
+                     nl->row_max.p, nl->stat_partial.p, s);
+      switch (G) {
+        case 1: PDX_ROWA(1) break;
+        case 2: PDX_ROWA(2) break;
+        case 4: PDX_ROWA(4) break;
+        case 8: PDX_ROWA(8) break;
+        case 16: PDX_ROWA(16) break;
+        default: PDX_ROWA(32) break;
+      }
+#undef PDX_ROWA
     } else if (cells) {
       row_blocks = std::min(nl->ncell, 8192);
 #define PDX_ROWC(GG)                                                                                        \
@@ -1271,9 +1384,9 @@ extern "C" int pdx_nl_create(int32_t n, const double box[3], double cutoff, doub
       (rc = nl->cell_offsets.alloc(nl->ncell + 1)) || (rc = nl->cell_counts.alloc(nl->ncell)) ||
       (rc = nl->particle_ids_sorted.alloc(n)) || (rc = nl->cell_of_particle.alloc(n)) ||
       (rc = nl->cell_rank.alloc(n)) || (rc = nl->rref.alloc((size_t)3 * n)) || (rc = nl->packed.alloc(n)) ||
-      (rc = nl->sorted.alloc(n)) || (rc = nl->sortedq.alloc(n)) || (rc = nl->disp_partial.alloc(nb)) || (rc = nl->row_max.alloc(1)) ||
+      (rc = nl->sorted.alloc(n)) || (rc = nl->sortedq.alloc(n)) || (rc = nl->disp_partial.alloc(nb)) || (rc = nl->row_max.alloc(ROW_CHOICE + 1)) ||
       (rc = nl->decision.alloc(sizeof(Decision) / sizeof(int64_t))) ||
-      (rc = nl->stat_partial.alloc((size_t)2 * cb)) || (rc = nl->scan_block.alloc(sblocks)) ||
+      (rc = nl->stat_partial.alloc((size_t)2 * cb)) || (rc = nl->scan_block.alloc(sblocks)) || (rc = nl->scan_occ.alloc(sblocks)) ||
       (rc = nl->candidates.alloc(nl->diagnostics ? n : 1)) ||
       (rc = nl->snap_offsets.alloc((size_t)nl->ncell + 1)) || (rc = nl->snap_ids.alloc(n)) ||
       (rc = nl->snap_state.alloc(4))) {
@@ -1485,7 +1598,8 @@ extern "C" int pdx_nl_set_box(pdx_nl_t nl, const double box[3], pdx_stream_t str
       PDX_HIP(hipStreamSynchronize(as_stream(stream)));
       const int ncell = g[0] * g[1] * g[2];
       if ((rc = nl->cell_offsets.alloc(ncell + 1)) || (rc = nl->cell_counts.alloc(ncell)) ||
-          (rc = nl->scan_block.alloc(blocks_for(ncell, SCAN_BLOCK))) || (rc = nl->snap_offsets.alloc(ncell + 1)))
+          (rc = nl->scan_block.alloc(blocks_for(ncell, SCAN_BLOCK))) ||
+          (rc = nl->scan_occ.alloc(blocks_for(ncell, SCAN_BLOCK))) || (rc = nl->snap_offsets.alloc(ncell + 1)))
         return rc;
       std::vector<int32_t> ones(ncell + 1, 1);
       PDX_HIP(hipMemcpy(nl->cell_offsets.p, ones.data(), sizeof(int32_t) * (ncell + 1), hipMemcpyHostToDevice));

@@ -344,3 +344,68 @@ def test_row_lanes_return_to_automatic(cuda):
     for bad in (-1, 3, 64):
         with pytest.raises(pdx.ArgumentError):
             eng.nl.set_row_lanes(bad)
+
+
+def _masks_pay(N, ncell, flat, used, largest):
+    """The library's choice of the cell-wise build, restated."""
+    if used < (2048 if flat else 1024) or largest * used > 2 * N + 16 * used:
+        return False
+    return N <= used * (100 if used >= 4096 or flat else 72 if used == ncell else 56)
+
+
+@pytest.mark.parametrize("kind,cellwise", [("uniform", True), ("dense corner", True), ("plane", True), ("sparse gas", False),
+                                           ("droplet", False), ("blob", False), ("crowded", False), ("thin plane", False)])
+def test_rows_of_uneven_cells_equal_row_search(cuda, kind, cellwise):
+    """The build chosen by how the particles fill the cells, on both sides of the choice, writes the rows of
+    the row search: even cells, cells of more particles than a wavefront with more candidates than one pass
+    holds, two-dimensional lists, a droplet, a blob in a gas."""
+    import torch
+    w, cutoff, skin = 3.001, 2.5, 0.5
+    rng = np.random.default_rng(len(kind))
+    flat = "plane" in kind
+    grid = {"plane": (46, 47), "thin plane": (44, 46), "sparse gas": (11, 11, 11)}.get(kind, (11, 12, 13))
+    box = tuple(w * g for g in grid)
+    B = np.array(box)
+    cells = int(np.prod(grid)) * (3 if flat else 1)
+
+    def gas(n, f=1.0):
+        return (rng.random((int(n), len(grid))) - 0.5) * B * f
+    if kind == "dense corner":  # 3 x 4 x 5 cells of 95 particles among cells of 60
+        p = gas(60 * cells)
+        q = (rng.random((60 * 35, 3)) * np.array([3, 4, 5]) + np.array([8, 8, 0])) * w - B / 2
+        p = np.concatenate([p, q])
+    elif kind == "droplet":
+        p = gas(15 * cells, 0.6)
+    elif kind == "blob":
+        p = np.concatenate([gas(13 * cells), gas(2 * cells, 0.15)])
+    else:
+        p = gas({"crowded": 90, "sparse gas": 14, "uniform": 20}.get(kind, 14.2) * cells)
+    if kind == "sparse gas":
+        p = p[(p ** 2).sum(1) > 19.0 ** 2]
+        p = np.concatenate([p, gas(14 * cells + 1 - len(p), 0.3)])
+    N = len(p)
+    p = np.clip(p.astype(np.float32), -np.float32(0.5) * B.astype(np.float32), np.float32(0.5) * B.astype(np.float32))
+    X = [dev(np.ascontiguousarray(p[:, d])) for d in range(len(grid))] + ([None] if flat else [])
+    for cap in (None, 30):
+        out = []
+        for lanes in (4, 0):
+            ws = pdx.DeviceNeighborWorkspace(N, box, cutoff, skin, cap or 30)
+            ws.set_row_lanes(lanes)
+            if cap is None:  # the capacity the first, failed build asks for
+                ws.update(*X, None)
+                ws.resize_capacity(max(30, ws.state()[8]))
+                ws.rearm()
+            print(f"[rows] {kind} N={N} cells={ws.ncell} cap={ws.cap} lanes={lanes}", flush=True)
+            ws.update(*X, None)
+            cnt, st = ws.counts().clone(), ws.state()
+            n = torch.diff(ws.cell_offsets().long())
+            used, largest = int((n > 0).sum()), int(n.max())
+            assert ws.ncell == cells and N >= 14 * cells
+            assert _masks_pay(N, cells, flat, used, largest) == cellwise, (used, largest)
+            keep = torch.arange(ws.cap, device="cuda")[:, None] < cnt[None, :]
+            out.append((cnt, torch.where(keep, ws.neighbors_flat(), torch.zeros_like(ws.neighbors_flat())), st))
+            del ws
+        (c0, r0, s0), (c1, r1, s1) = out
+        assert torch.equal(c0, c1) and torch.equal(r0, r1)
+        assert s0 == s1
+        assert (int(c0.max()) > r0.shape[0]) == (s0[2] != 0)
