@@ -143,10 +143,24 @@ __device__ __forceinline__ int wave_max(int v) {
   for (int off = 32; off >= 1; off >>= 1) v = max(v, __shfl_xor(v, off, WAVE));
   return v;
 }
-__device__ __forceinline__ int wave_min(int v) {
+// Least and greatest n of a wave whose lanes hold one in groups of G (every lane active): lane exchanges
+// in the vector unit up to the rows of 16 lanes, then scalars; no trip through LDS.
+template <int G>
+__device__ __forceinline__ int2 wave_range(int n) {
+  int lo = n, hi = n;
+#define PDX_STEP(ctrl)                                                        \
+  lo = min(lo, __builtin_amdgcn_mov_dpp(lo, ctrl, 0xf, 0xf, true));           \
+  hi = max(hi, __builtin_amdgcn_mov_dpp(hi, ctrl, 0xf, 0xf, true));
+  if (G < 2) { PDX_STEP(0xB1) }    // quad_perm: the other lane of a pair
+  if (G < 4) { PDX_STEP(0x4E) }    // quad_perm: the other pair of a quad
+  if (G < 8) { PDX_STEP(0x141) }   // row_half_mirror: the other quad of eight lanes
+  if (G < 16) { PDX_STEP(0x140) }  // row_mirror: the other half of a row
+#undef PDX_STEP
+  int2 r = make_int2(__builtin_amdgcn_readlane(lo, 0), __builtin_amdgcn_readlane(hi, 0));
 #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v = min(v, __shfl_xor(v, off, WAVE));
-  return v;
+  for (int l = G < 16 ? 16 : G; l < WAVE; l += G < 16 ? 16 : G)
+    r = make_int2(min(r.x, __builtin_amdgcn_readlane(lo, l)), max(r.y, __builtin_amdgcn_readlane(hi, l)));
+  return r;
 }
 __device__ __forceinline__ float wave_max(float v) {
 #pragma unroll

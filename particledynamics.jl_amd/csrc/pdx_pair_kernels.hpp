@@ -132,8 +132,9 @@ __device__ __forceinline__ void walk_rows(const PairArgs &a, const float4 &pi, i
     visit(jj, pj, dx, dy, dz);
   };
   const int32_t *row = a.nbr + i;
-  const int full = WIDE ? 0 : __builtin_amdgcn_readfirstlane(wave_min(n) / (U * G));
-  const int its = __builtin_amdgcn_readfirstlane((wave_max(n) + U * G - 1) / (U * G));
+  const int2 range = wave_range<G>(n);
+  const int full = WIDE ? 0 : range.x / (U * G);
+  const int its = (range.y + U * G - 1) / (U * G);
   const int vo = (int)walk_lane(lane, N, i);
   auto load = [&](int k, int (&id)[U]) {
     if (k < full) {
