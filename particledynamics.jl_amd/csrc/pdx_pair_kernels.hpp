@@ -161,11 +161,23 @@ __device__ __forceinline__ void walk_rows(const PairArgs &a, const float4 &pi, i
   }
 }
 
+// Waves a SIMD that the row kernels are held to. The row loop waits for its gathers, so it is the highest
+// number that leaves the loop without scratch accesses: forces only 8 (64 registers), with energies 6 (80),
+// less where the Coulomb polynomials meet per-pair coefficients or one lane's longer index arithmetic.
+// Spilled at 8, pair matrices with Coulomb took 13.1 us (20 000 particles, forces) and 24.8 us (64 000),
+// mixed diameters 11.6 and 20.8 us; at 7 waves 10.5 and 20.1, 9.5 and 18.5 us.
+__host__ __device__ constexpr int pair_waves(int model, bool coul, bool energy, int G, int NP) {
+  const bool typed = typed_model(model), soft = model == PDX_PAIR_SOFT;
+  if (energy) return coul && G == 1 && (typed || (soft && NP > 16)) ? 5 : 6;
+  if (G == 1) return coul && typed ? 6 : (coul || typed ? 7 : 8);
+  return coul && (typed || soft) ? 7 : 8;
+}
+
 // Layout A: G lanes of one wave per particle, xor-shuffle reduction. Forces-only launches evaluate
 // every pair with pair_terms in row order (the sums are then the same bits whatever the traversal's
 // bookkeeping, which trajectories keep); energy launches use the joined terms.
 template <int MODEL, bool COUL, bool ENERGY, int G, int NP, bool WIDE = false>
-__global__ __launch_bounds__(TPB, ENERGY ? 6 : 8) void k_pair(const PairArgs a) {
+__global__ __launch_bounds__(TPB, pair_waves(MODEL, COUL, ENERGY, G, NP)) void k_pair(const PairArgs a) {
   const int64_t *s = a.state;
   const bool valid = s[PDX_DN_VALID] != 0 && s[PDX_DN_ERROR] == 0;  // uniform
   if (!valid) return;
@@ -605,7 +617,7 @@ template <> struct Sum<PDX_ACC_FP64> {
 };
 
 template <int MODEL, bool ENERGY, int G, int ACC, bool WIDE = false>
-__global__ __launch_bounds__(TPB, ACC == PDX_ACC_FP32 ? 6 : 1) void k_pair_acc(const PairArgs a, int bonded) {
+__global__ __launch_bounds__(TPB, ACC == PDX_ACC_FP32 ? (ENERGY ? 6 : 7) : 1) void k_pair_acc(const PairArgs a, int bonded) {
   const int64_t *s = a.state;
   const bool valid = s[PDX_DN_VALID] != 0 && s[PDX_DN_ERROR] == 0;  // uniform
   if (!valid) return;
