@@ -771,12 +771,12 @@ __global__ __launch_bounds__(TPB) void k_rows_cells(int N, int cap, int ncell, i
   row_partials(longest, all_tested, all_found, row_max, stat_partial);
 }
 
-// ---- the build of many evenly filled cells: one workgroup per cell, lanes = candidates,
-// particles one after the other in scalar registers (four waves, a chunk of 64 candidates each in
-// turn). A distance test of 64 candidates is then seven vector instructions (three more per
-// dimension where the stencil crosses the seam), its ballot goes into lane p of a register pair (particle p of the cell), and the cell's tests end as bit
-// masks in LDS. The rows are written in a second pass with lanes = particles, each wave a quarter of
-// the masks from the slot its earlier ones add up to: every lane takes its next set bit, so a store
+// ---- the build of many evenly filled cells: one workgroup per cell, lanes = candidates, particles one
+// after the other in scalar registers (four waves, a chunk of 64 candidates each in turn). A distance test
+// of 64 candidates is then seven vector instructions (three more per dimension where the stencil crosses
+// the seam), its ballot goes into lane p of a register pair (particle p of the cell), and the cell's tests
+// end as bit masks in LDS. The rows are written in a second pass with lanes = particles, each wave a quarter
+// of the masks from the slot its earlier ones add up to: every lane takes its next set bit, so a store
 // writes neighbouring slots of the cell's rows, lines that fill up within a few steps where the
 // cell's particles are contiguous in storage (spatial order). Candidates are numbered in stencil
 // order (z, y, x cells, then the cells' order), so rows are k_rows' rows.
@@ -784,9 +784,10 @@ __global__ __launch_bounds__(TPB) void k_rows_cells(int N, int cap, int ncell, i
 // writes). k_rows spends 38 on 64 tests (per-lane image, ballots, predicated 4-byte stores that each
 // touch their own line). Whole rebuilds with it at its best lane count and with this kernel: 326 and
 // 264 us (256 000 LJ atoms, 21 a cell), 1 224 and 1 020 us (486 400 ions, 61 a cell).
-// v_writelane_b32 (this compiler has the intrinsic but no builtin for it): old with lane `lane` = value,
-// both uniform.
-extern "C" __device__ __attribute__((const)) int pdx_writelane(int value, int lane, int old) __asm("llvm.amdgcn.writelane.i32");
+// v_writelane_b32: old with lane `lane` = value, both uniform. This compiler has the intrinsic but no
+// builtin for it; a compiler without it refuses the name.
+extern "C" __device__ __attribute__((const)) int pdx_writelane(int value, int lane,
+                                                               int old) __asm("llvm.amdgcn.writelane.i32");
 constexpr int RM_CHUNKS = 28;  // candidate chunks of 64 per pass (21 KiB of LDS: seven workgroups per CU)
 constexpr int RM_WAVES = TPB / WAVE;
 __device__ __forceinline__ void mask_rows(int N, int cap, int ncell, int nx, int ny, int nz,
@@ -1148,9 +1149,12 @@ int enqueue_decide_build(pdx_nl_t nl, hipStream_t st) {
   const float threshold = (0.25f * skin) * skin;
   int row_blocks = nb;  // workgroups of the row kernel, one commit partial each
   // k_bin decides where its workgroups reread at most 1 024 partials each (4 KB, from the caches) and
-  // k_scan_scatter follows to write the decision down; else a launch of its own does. Forty steps of
-  // 256 000 LJ atoms (1 000 blocks): 3.67 ms in k_bin, 3.74 apart; a pass of 7 600 ions 78 and 82 us;
-  // forty steps of 486 400 ions (1 900 blocks, beside the mesh): 23.2 ms in k_bin, 22.9 apart
+  // k_scan_scatter follows to write the decision down; else a launch of its own does. Forty steps in
+  // k_bin and apart: LJ atoms 6 912 1.15 and 1.22 ms, 62 500 1.79 and 1.87, 256 000 (1 000 blocks) 3.68 and
+  // 3.74, 500 000 6.13 both; ions beside a mesh 27 000 4.64 and 4.66, 64 000 5.14 and 5.17, 262 144 (1 024
+  // blocks) 22.23 and 22.14, 486 400 23.2 and 22.9. Single evaluations beside a mesh: 7 600 ions 78 and
+  // 82 us, 64 000 124 and 125.5. (With the scan apart too, 64 000 ions take 123 us, but 5.24 ms for forty
+  // steps: the chain's launches then end after the spread instead of beside it.)
   const bool scan_fused = !nl->allpairs && nl->ncell <= SCAN_FUSED_MAX;
   const bool decide_fused = scan_fused && nb <= DECIDE_BLOCKS;
   Decision *dec = (Decision *)nl->decision.p;
@@ -1282,12 +1286,14 @@ int enqueue_check(pdx_nl_t nl, const float *x, const float *y, const float *z, c
   float *xw = const_cast<float *>(x), *yw = const_cast<float *>(y), *zw = const_cast<float *>(z);
   if (kd)
     hipLaunchKernelGGL(k_decide<true>, dim3(nb), dim3(TPB), 0, st, N, xw, yw, zw, q, nl->rref.p, nl->packed.p,
-                       nl->cell_counts.p, nl->row_max.p, nl->ncell, (int)nl->allpairs, nl->geom.p, nl->state.p, nl->disp_partial.p,
+                       nl->cell_counts.p, nl->row_max.p, nl->ncell, (int)nl->allpairs, nl->geom.p, nl->state.p,
+                       nl->disp_partial.p,
                        (const int32_t *)nl->cell_offsets.p, (const int32_t *)nl->particle_ids_sorted.p,
                        nl->snap_offsets.p, nl->snap_ids.p, nl->snap_state.p, *kd);
   else
     hipLaunchKernelGGL(k_decide<false>, dim3(nb), dim3(TPB), 0, st, N, xw, yw, zw, q, nl->rref.p, nl->packed.p,
-                       nl->cell_counts.p, nl->row_max.p, nl->ncell, (int)nl->allpairs, nl->geom.p, nl->state.p, nl->disp_partial.p,
+                       nl->cell_counts.p, nl->row_max.p, nl->ncell, (int)nl->allpairs, nl->geom.p, nl->state.p,
+                       nl->disp_partial.p,
                        (const int32_t *)nl->cell_offsets.p, (const int32_t *)nl->particle_ids_sorted.p,
                        nl->snap_offsets.p, nl->snap_ids.p, nl->snap_state.p, KickDrift{});
   PDX_LAUNCH_CHECK();
@@ -1384,9 +1390,11 @@ extern "C" int pdx_nl_create(int32_t n, const double box[3], double cutoff, doub
       (rc = nl->cell_offsets.alloc(nl->ncell + 1)) || (rc = nl->cell_counts.alloc(nl->ncell)) ||
       (rc = nl->particle_ids_sorted.alloc(n)) || (rc = nl->cell_of_particle.alloc(n)) ||
       (rc = nl->cell_rank.alloc(n)) || (rc = nl->rref.alloc((size_t)3 * n)) || (rc = nl->packed.alloc(n)) ||
-      (rc = nl->sorted.alloc(n)) || (rc = nl->sortedq.alloc(n)) || (rc = nl->disp_partial.alloc(nb)) || (rc = nl->row_max.alloc(ROW_CHOICE + 1)) ||
+      (rc = nl->sorted.alloc(n)) || (rc = nl->sortedq.alloc(n)) || (rc = nl->disp_partial.alloc(nb)) ||
+      (rc = nl->row_max.alloc(ROW_CHOICE + 1)) ||
       (rc = nl->decision.alloc(sizeof(Decision) / sizeof(int64_t))) ||
-      (rc = nl->stat_partial.alloc((size_t)2 * cb)) || (rc = nl->scan_block.alloc(sblocks)) || (rc = nl->scan_occ.alloc(sblocks)) ||
+      (rc = nl->stat_partial.alloc((size_t)2 * cb)) || (rc = nl->scan_block.alloc(sblocks)) ||
+      (rc = nl->scan_occ.alloc(sblocks)) ||
       (rc = nl->candidates.alloc(nl->diagnostics ? n : 1)) ||
       (rc = nl->snap_offsets.alloc((size_t)nl->ncell + 1)) || (rc = nl->snap_ids.alloc(n)) ||
       (rc = nl->snap_state.alloc(4))) {

@@ -174,8 +174,8 @@ __host__ __device__ constexpr int pair_waves(int model, bool coul, bool energy, 
 }
 
 // Layout A: G lanes of one wave per particle, xor-shuffle reduction. Forces-only launches evaluate
-// every pair with pair_terms in row order (the sums are then the same bits whatever the traversal's
-// bookkeeping, which trajectories keep); energy launches use the joined terms.
+// every pair with pair_terms in row order (at a given lane count the sums are then the same bits whatever
+// the traversal's bookkeeping, which trajectories keep); energy launches use the joined terms.
 template <int MODEL, bool COUL, bool ENERGY, int G, int NP, bool WIDE = false>
 __global__ __launch_bounds__(TPB, pair_waves(MODEL, COUL, ENERGY, G, NP)) void k_pair(const PairArgs a) {
   const int64_t *s = a.state;
@@ -581,9 +581,9 @@ void launch_cells(bool coul, bool energy, int np, dim3 grid, hipStream_t st, con
 }
 
 // ---- per-particle sums in a chosen precision (the bead-spring precision study). The pair
-// arithmetic is the FP32 arithmetic of k_pair; only the accumulation of the row sums changes:
-// FP32 (fma, as k_pair), 64-bit fixed point at 2^32 (exact, so independent of the order and of
-// the lane split), or FP64 (exact products, rounded sums).
+// arithmetic is that of k_pair's forces-only launches (pair_terms in FP32), with energies too; only the
+// accumulation of the row sums changes: FP32 (fma, as k_pair), 64-bit fixed point at 2^32 (exact, so
+// independent of the order and of the lane split), or FP64 (exact products, rounded sums).
 template <int ACC> struct Sum;
 template <> struct Sum<PDX_ACC_FP32> {
   float v = 0.f;
@@ -617,7 +617,8 @@ template <> struct Sum<PDX_ACC_FP64> {
 };
 
 template <int MODEL, bool ENERGY, int G, int ACC, bool WIDE = false>
-__global__ __launch_bounds__(TPB, ACC == PDX_ACC_FP32 ? (ENERGY ? 6 : 7) : 1) void k_pair_acc(const PairArgs a, int bonded) {
+__global__ __launch_bounds__(TPB, ACC == PDX_ACC_FP32 ? (ENERGY ? 6 : 7) : 1) void k_pair_acc(const PairArgs a,
+                                                                                             int bonded) {
   const int64_t *s = a.state;
   const bool valid = s[PDX_DN_VALID] != 0 && s[PDX_DN_ERROR] == 0;  // uniform
   if (!valid) return;
@@ -743,7 +744,8 @@ __global__ __launch_bounds__(TPB, ACC == PDX_ACC_FP32 ? (ENERGY ? 6 : 7) : 1) vo
 }
 
 template <int MODEL, bool ENERGY, int ACC>
-void launch_acc_g(int G /* 0: one lane, 64-bit addresses */, dim3 grid, hipStream_t st, const PairArgs &a, int bonded) {
+void launch_acc_g(int G /* 0: one lane, 64-bit addresses */, dim3 grid, hipStream_t st, const PairArgs &a,
+                  int bonded) {
   switch (G) {
     case 0: hipLaunchKernelGGL((k_pair_acc<MODEL, ENERGY, 1, ACC, true>), grid, dim3(TPB), 0, st, a, bonded); break;
     case 1: hipLaunchKernelGGL((k_pair_acc<MODEL, ENERGY, 1, ACC>), grid, dim3(TPB), 0, st, a, bonded); break;

@@ -1,5 +1,7 @@
-// Per-pair physics shared by the ELL-row and cluster-tile traversals: the model terms of one
-// pair at squared distance r2, so both traversals evaluate every pair identically.
+// Per-pair physics shared by the row, cell and cluster-tile traversals: the model terms of one pair at
+// squared distance r2. Every traversal evaluates pair_terms (typed models pair_terms_c), except the rows'
+// energy launches of uniform models with FP32 sums, which take pair_terms_joint: the same terms up to
+// rounding.
 #pragma once
 
 #include "pdx_internal.hpp"

@@ -274,7 +274,10 @@ int pair_forces_impl(pdx_pair_t p, pdx_nl_t nl, float *fx, float *fy, float *fz,
     // particle gather from the same few cells, so a wave touches 16 rows' neighbourhoods instead of
     // 64 (256 000 LJ atoms, 82 entries: 58 -> 40 us; 512 000 ions, 187 entries: 423 -> 304 us, with
     // 2 lanes 46 and 338, with 8 lanes 45 and 310). Short rows leave such lanes idle (1 M beads, 14
-    // entries: 60 us with one lane, 76 with four), and the accumulation modes keep their split.
+    // entries: 60 us with one lane, 76 with four), and the accumulation modes keep their split. Around
+    // the line, 500 000 LJ atoms with one and four lanes: 19 entries 23.4 and 21.6 us (forces) and 35.5
+    // and 44.3 (energies), 33 entries 39.9 and 30.1, 52.2 and 50.6; LJ + Coulomb energies cross later,
+    // 33 entries 57.7 and 63.0, 42 entries 63.4 and 63.5, 54 entries 76.6 and 75.8.
     const double rl = std::sqrt((double)nl->rl2);
     const double rows = 4.1887902 * rl * rl * rl * N / (nl->box[0] * nl->box[1] * nl->box[2]);
     if (!acc_path && rows >= 32.0) G = std::max(G, 4);
