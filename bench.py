@@ -150,7 +150,27 @@ def main():
     if not args.no_cpu_baseline:
         _log("CPU baseline")
         out["cpu_baseline"] = cpu_baseline(head["sysd"], head["plain_spec"])
+    print(json.dumps({"tables": take_tables(out)}), file=sys.stderr, flush=True)
     print(json.dumps(out))
+
+
+def take_tables(out):
+    """The searches' and tuners' tables of the comparisons, taken out of the line (they make it longer than
+    a reader that keeps the last 16 KB of the output can see)."""
+    tables = {}
+    for name, line in (("headline", out), ("learned_60800", out.get("learned_60800"))):
+        c = (line or {}).get("comparison")
+        if not c:
+            continue
+        t = tables[name] = {"plain_search": c.pop("plain_search", None), "candidates": {}}
+        for key, tuned in (c.get("autotune") or {}).items():
+            t["candidates"][key] = tuned.pop("candidates", None)
+        f = c.get("frontier") or {}
+        t["frontier_plain"], t["frontier_plain_pareto"] = f.pop("plain", None), f.pop("plain_pareto", None)
+    for name, leg in (out.get("published_coulomb") or {}).items():
+        if isinstance(leg, dict) and "errors_by_order_and_tolerance" in leg:
+            tables[name] = leg.pop("errors_by_order_and_tolerance")
+    return tables
 
 
 C_ION = 14.399645

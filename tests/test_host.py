@@ -87,3 +87,20 @@ def test_autotune_classes_and_table(tmp_path):
     assert autotune.settings_for(64000, (112.8,) * 3, 9.0, True, table=t)["force_lanes"] == 4
     assert autotune.settings_for(64000, (112.8,) * 3, 9.0, False, table=t) is None
     assert autotune.load(str(tmp_path / "missing.json")) == {}
+
+
+def test_bench_line_leaves_its_tables_out():
+    """The searches' and tuners' tables are taken out of the benchmark's line, the best settings stay."""
+    import json
+    import bench
+    comparison = {"plain_search": [{"rc": 9.0}] * 400, "speedup": 2.0,
+                  "autotune": {"a": {"best": {"force_lanes": 4}, "candidates": [[{"force_lanes": 1}, 0.5]] * 400}},
+                  "frontier": {"plain": [{"err": 1e-4}] * 400, "plain_pareto": [1] * 400}}
+    out = {"metric": "m", "value": 1.0, "comparison": comparison,
+           "published_coulomb": {"note": "n", "SPME": {"N": 1, "errors_by_order_and_tolerance": {"P": [1.0] * 400}}},
+           "learned_60800": {"comparison": json.loads(json.dumps(comparison))}}
+    tables = bench.take_tables(out)
+    assert len(json.dumps(out)) < 600 and len(tables["headline"]["plain_search"]) == 400
+    assert len(tables["learned_60800"]["candidates"]["a"]) == 400 and len(tables["headline"]["frontier_plain"]) == 400
+    assert out["comparison"]["autotune"]["a"]["best"] == {"force_lanes": 4}
+    assert bench.take_tables({"metric": "m"}) == {}
