@@ -225,11 +225,10 @@ def test_rows_staged_equal_direct_and_lanes(cuda, case, monkeypatch):
 @pytest.mark.parametrize("grid", [(3, 18, 20), (4, 16, 17), (5, 14, 15), (10, 11, 12)])
 @pytest.mark.parametrize("clump", [0, 2200])
 def test_rows_of_dense_cells_equal_row_search(cuda, grid, clump):
-    """The cell-wise build that many well-filled cells take by default (at least 1 024 cells of 14
-    particles and more) writes the rows, slot for slot, the candidate counts and the statistics of the
-    row search (an explicit lane count): grids with and without cells off the seam, particles on the
-    box faces, a clump with more particles in a cell than a wavefront has lanes and more candidates
-    than one pass holds, and rows longer than the capacity."""
+    """The automatic build of at least 1 024 cells of 14 particles and more writes the rows, slot for slot,
+    the candidate counts and the statistics of the row search (an explicit lane count): cell-wise on grids
+    with and without cells off the seam and particles on the box faces, by the search with a clump of more
+    particles in a cell than a wavefront has lanes; and rows longer than the capacity."""
     import torch
     w, cutoff, skin = 3.001, 2.5, 0.5
     box = tuple(w * g for g in grid)
